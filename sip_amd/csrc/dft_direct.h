@@ -1,0 +1,52 @@
+// Element loads and stores shared by the kernels that take DftArgs (dft_unit_kernel,
+// bluestein_kernel): every prologue / epilogue as a uniform run-time branch, since these kernels
+// are compiled once per length and not per layout.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "fft_kernel_args.h"
+
+namespace asdfft {
+
+__device__ __forceinline__ float2 dft_load(const DftArgs& a, int64_t base, int i)
+{
+    const float2* in2 = reinterpret_cast<const float2*>(a.in);
+    const int64_t s = a.in_stride;
+    float2 x;
+    if (a.prologue == kProReal) {
+        x = make_float2(reinterpret_cast<const float*>(a.in)[base + i * s], 0.0f);
+    } else if (a.prologue == kProPlanar) {
+        x = make_float2(reinterpret_cast<const float*>(a.in)[base + i * s], a.in_im[base + i * s]);
+    } else if (a.prologue == kProHerm) {
+        const int h = a.n >> 1;
+        if (i <= h) {
+            x = in2[base + i * s];
+            if (i == 0 || 2 * i == a.n) x.y = 0.0f;
+        } else {
+            x = in2[base + (a.n - i) * s];
+            x.y = -x.y;
+        }
+    } else {
+        x = in2[base + i * s];
+    }
+    if (a.conj_in) x.y = -x.y;
+    return x;
+}
+
+__device__ __forceinline__ void dft_store(const DftArgs& a, int64_t base, int k, float2 x)
+{
+    if (a.epilogue == kEpiReal) {
+        reinterpret_cast<float*>(a.out)[base + k] = x.x;
+        return;
+    }
+    if (a.conj_out) x.y = -x.y;
+    if (a.epilogue == kEpiPlanar) {
+        reinterpret_cast<float*>(a.out)[base + k] = x.x;
+        a.out_im[base + k] = x.y;
+    } else if (a.epilogue != kEpiHalf || 2 * k <= a.n) {
+        reinterpret_cast<float2*>(a.out)[base + k] = x;
+    }
+}
+
+}  // namespace asdfft

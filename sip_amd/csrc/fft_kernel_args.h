@@ -121,14 +121,19 @@ struct RaggedArgs {
     int ntiles;
 };
 
-// Direct O(N^2) DFT kernel parameters (lengths with factors outside the radix set, N == 1).
+// Transforms of lengths with factors outside the radix set (chirp transform, bluestein.hip; sum
+// over pairs at 23, 29, 31) and of length 1.
 struct DftArgs {
     const void* in;
     void* out;
     const float* in_im;     // planar input / output planes (kProPlanar, kEpiPlanar)
     float* out_im;
-    const float* roots;     // W_N^m, m in [0, N)
+    const float* roots;     // chirp e^(-i pi k^2 / n), k in [0, n); sum over pairs: W_n^k
+    const float* filter;    // M-point transform of the conjugate chirp, over M
+    const float* tw_first;  // per-pass twiddles of the first / second M-point transform
+    const float* tw_second;
     int n;
+    int m;                  // convolution length M
     int tpb;
     int conj_in, conj_out;
     int prologue, epilogue; // kProComplex/kProReal/kProHerm/kProPlanar, kEpiComplex/kEpiHalf/kEpiReal/kEpiPlanar

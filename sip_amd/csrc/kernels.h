@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <stdint.h>
+#include <vector>
 
 #include "fft_kernel_args.h"
 
@@ -20,7 +21,7 @@ enum Variant : int {
     kVarC2ROdd = 5,
     kVarColsTwiddle = 6,
     kVarRowsTranspose = 7,
-    kVarDirect = 8,  // dft_direct_kernel
+    kVarDirect = 8,  // bluestein_kernel, dft_pairs_kernel, dft_unit_kernel
     // separated real/imaginary planes (ASCEND_FFT_C2C_SEP plans)
     kVarRowsSep = 9,            // rows, planar in and out
     kVarRowsSepIn = 10,         // rows, planar in, complex out
@@ -85,6 +86,11 @@ extern const int kNumStaticInstances;
 // for the column mapping (rows keep transforms-per-workgroup at run time).
 int find_static(int variant, int emax, int n, int threads, int tpb, const int* radices, int nradices);
 hipError_t launch_dft_direct(const LaunchShape& s, const DftArgs& args, hipStream_t stream);
+bool dft_pairs_length(int64_t n);  // 23, 29, 31: the sum over pairs (dft_pairs_kernel)
+int dft_pairs_per_block();
+hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, hipStream_t stream);
+// Radices of the first / second transform of convolution length m (empty: no kernel).
+std::vector<int> bluestein_radices(int64_t m, bool second);
 hipError_t launch_istft_ola(const OlaArgs& args, hipStream_t stream);
 hipError_t launch_real_aux(const RealAuxArgs& args, hipStream_t stream);
 

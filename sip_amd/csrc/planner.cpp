@@ -510,22 +510,19 @@ bool attach_aux(Step* st, int64_t nreal)
     return true;
 }
 
+// Length 1, and lengths with prime factors above 19: the sum over pairs at 23, 29 and 31, the
+// chirp transform (bluestein.hip) above.
 bool direct_step(int64_t n, int prologue, int epilogue, int64_t count, int64_t in_dist, int64_t out_dist, int conj_in,
                  int conj_out, Step* st, std::string* why)
 {
     if (n > kMaxDirect) {
-        *why = "length " + std::to_string(n) + " has prime factors above 19 and exceeds the direct-DFT limit";
+        *why = "length " + std::to_string(n) + " has prime factors above 19 and exceeds the chirp transform's limit";
         return false;
     }
-    TablePtr t = upload_table("roots:" + std::to_string(n), roots_table(n, n));
-    st->tables_ready = (t != nullptr);
-    if (t) st->tables.push_back(t);
     DftArgs& d = st->dargs;
     d = DftArgs{};
-    d.roots = t ? t->dev : nullptr;
     d.n = (int)n;
-    int tpb = (int)std::max<int64_t>(1, std::min<int64_t>(count, std::max<int64_t>(1, 4096 / n)));
-    d.tpb = tpb;
+    d.tpb = 256;
     d.conj_in = conj_in;
     d.conj_out = conj_out;
     d.prologue = prologue;
@@ -536,13 +533,55 @@ bool direct_step(int64_t n, int prologue, int epilogue, int64_t count, int64_t i
     d.in_cols = 1;
     d.in_stride = 1;
     st->direct = true;
+    st->tables_ready = device_available();
     st->shape.variant = kVarDirect;
     st->shape.emax = 0;
     st->shape.block = 256;
-    st->shape.lds_bytes = (size_t)tpb * (size_t)n * 8;
-    st->shape.grid = (count + tpb - 1) / tpb;
     std::ostringstream os;
-    os << "direct n=" << n << " count=" << count << " pro=" << prologue << " epi=" << epilogue << " tpb=" << tpb;
+    os << "direct n=" << n << " count=" << count << " pro=" << prologue << " epi=" << epilogue;
+    auto use = [&](const TablePtr& t) -> const float* {
+        if (!t) {
+            st->tables_ready = false;
+            return nullptr;
+        }
+        st->tables.push_back(t);
+        return t->dev;
+    };
+    if (dft_pairs_length(n)) {
+        d.tpb = dft_pairs_per_block();
+        d.roots = use(upload_table("roots:" + std::to_string(n), roots_table(n, n)));
+        os << " pairs";
+    } else if (n > 1) {
+        int64_t m = 128;
+        while (m < 2 * n - 1) m *= 2;
+        const std::vector<int> first = bluestein_radices(m, false), second = bluestein_radices(m, true);
+        if (first.empty()) {
+            *why = "no chirp transform of length " + std::to_string(n);
+            return false;
+        }
+        d.m = (int)m;
+        auto passes = [&](const std::vector<int>& radices) {
+            return use(upload_table(radix_key(m, radices), [&] {
+                std::vector<int> offsets;
+                return stockham_table((int)m, radices, &offsets);
+            }));
+        };
+        d.tw_first = passes(first);
+        d.tw_second = (second == first) ? d.tw_first : passes(second);
+        d.roots = use(upload_table("chirp:" + std::to_string(n), [&] { return chirp_table(n); }));
+        d.filter = use(upload_table("chirpfilter:" + std::to_string(n) + ":" + std::to_string(m),
+                                    [&] { return chirp_filter_table(n, m); }));
+        // several short transforms per workgroup of 256 threads; fewer in a small batch, so that it
+        // spreads over two workgroups per CU, but at least one full wavefront
+        const int64_t T = m / 16;
+        const int64_t spread = std::max<int64_t>((64 + T - 1) / T, count / (2 * kNumCUs));
+        d.tpb = (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / T, spread), count));
+        st->shape.block = (int)(d.tpb * T);
+        st->shape.lds_bytes = (size_t)d.tpb * (size_t)(m + m / 16 + 1) * 8;
+        os << " chirp m=" << m;
+    }
+    st->shape.grid = (count + d.tpb - 1) / d.tpb;
+    os << " tpb=" << d.tpb << " grid=" << st->shape.grid;
     st->describe = os.str();
     return true;
 }

@@ -26,7 +26,7 @@ enum class Kind { C2C, R2C, C2R };
 
 // Largest complex length one workgroup transforms (all of it resident in LDS).
 constexpr int64_t kMaxSingleKernel = 16384;
-// Largest length the O(N^2) direct kernel accepts (lengths with prime factors > 19).
+// Largest length with prime factors above 19 (chirp transform, one workgroup).
 constexpr int64_t kMaxDirect = 8192;
 
 struct Schedule {

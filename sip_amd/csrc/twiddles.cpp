@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <complex>
 #include <map>
 #include <mutex>
 
@@ -57,6 +58,59 @@ std::vector<float> stockham_table(int n, const std::vector<int>& radices, std::v
     return tab;
 }
 
+static const double kPi = 3.14159265358979323846;
+
+// angle of the chirp at k, reduced exactly
+static double chirp_angle(int64_t n, int64_t k) { return kPi * (double)((k * k) % (2 * n)) / (double)n; }
+
+std::vector<float> chirp_table(int64_t n)
+{
+    std::vector<float> out(2 * (size_t)n);
+    for (int64_t k = 0; k < n; k++) {
+        const double ang = chirp_angle(n, k);
+        out[2 * k] = (float)cos(ang);
+        out[2 * k + 1] = (float)(-sin(ang));
+    }
+    return out;
+}
+
+std::vector<float> chirp_filter_table(int64_t n, int64_t m)
+{
+    std::vector<std::complex<double>> x((size_t)m), root((size_t)m / 2);
+    for (int64_t k = 0; k < n; k++) {
+        const double ang = chirp_angle(n, k);
+        x[(size_t)k] = {cos(ang), sin(ang)};
+        if (k > 0) x[(size_t)(m - k)] = x[(size_t)k];
+    }
+    for (int64_t k = 0; k < m / 2; k++) {
+        const double ang = 2.0 * kPi * (double)k / (double)m;
+        root[(size_t)k] = {cos(ang), -sin(ang)};
+    }
+    auto mul = [](std::complex<double> a, std::complex<double> b) {  // finite factors: no NaN recovery
+        return std::complex<double>(a.real() * b.real() - a.imag() * b.imag(),
+                                    a.real() * b.imag() + a.imag() * b.real());
+    };
+    // radix-2 decimation in frequency in double; the result comes out bit-reversed
+    for (int64_t half = m / 2; half >= 1; half /= 2) {
+        const int64_t step = (m / 2) / half;
+        for (int64_t base = 0; base < m; base += 2 * half) {
+            for (int64_t j = 0; j < half; j++) {
+                const std::complex<double> u = x[(size_t)(base + j)], v = x[(size_t)(base + j + half)];
+                x[(size_t)(base + j)] = u + v;
+                x[(size_t)(base + j + half)] = mul(u - v, root[(size_t)(j * step)]);
+            }
+        }
+    }
+    std::vector<float> out(2 * (size_t)m);
+    for (int64_t k = 0; k < m; k++) {
+        int64_t r = 0;
+        for (int64_t bit = 1, b = k; bit < m; bit *= 2, b /= 2) r = 2 * r + (b & 1);
+        out[2 * r] = (float)(x[(size_t)k].real() / (double)m);
+        out[2 * r + 1] = (float)(x[(size_t)k].imag() / (double)m);
+    }
+    return out;
+}
+
 bool device_available()
 {
     static int state = -1;  // -1 unknown, 0 no, 1 yes
@@ -72,6 +126,11 @@ bool device_available()
 
 TablePtr upload_table(const std::string& key, const std::vector<float>& host)
 {
+    return upload_table(key, [&] { return host; });
+}
+
+TablePtr upload_table(const std::string& key, const std::function<std::vector<float>()>& generate)
+{
     if (!device_available()) return nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -82,6 +141,7 @@ TablePtr upload_table(const std::string& key, const std::vector<float>& host)
     if (it != cache.end()) {
         if (TablePtr p = it->second.lock()) return p;
     }
+    const std::vector<float> host = generate();
     auto t = std::make_shared<DeviceTable>();
     t->device = dev;
     t->entries = host.size() / 2;
