@@ -65,7 +65,7 @@ inline hipError_t raise_lds_limit_once(const void* fn, std::atomic<uint64_t>& ra
 struct LaunchShape {
     int static_id = -1;  // index into kStaticInstances, or -1 for the run-time kernel
     int variant;
-    int emax;          // registers per thread (complex points): 16, 32 or 48
+    int emax;          // registers per thread (complex points): 16 or 32 (64: specialised only)
     int block;         // threads per workgroup
     size_t lds_bytes;  // dynamic LDS
     int64_t grid;      // workgroups
@@ -101,12 +101,10 @@ hipError_t launch_real_aux(const RealAuxArgs& args, hipStream_t stream);
 #define ASDFFT_FOR_EACH_INSTANCE(X) \
     X(0, 16) X(1, 16) X(2, 16) X(3, 16) X(4, 16) X(5, 16) X(6, 16) X(7, 16) \
     X(0, 32) X(1, 32) X(2, 32) X(3, 32) X(4, 32) X(5, 32) X(6, 32) X(7, 32) \
-    X(0, 48) X(1, 48) X(2, 48) X(3, 48) X(4, 48) X(5, 48) \
     X(9, 16) X(10, 16) X(11, 16) X(12, 16) X(13, 16) \
     X(9, 32) X(10, 32) X(11, 32) X(12, 32) X(13, 32) \
-    X(9, 48) X(10, 48) X(11, 48) \
     X(14, 16) X(14, 32) \
-    X(16, 16) X(17, 16) X(18, 16) X(16, 32) X(17, 32) X(18, 32) X(16, 48) X(17, 48)
+    X(16, 16) X(17, 16) X(18, 16) X(16, 32) X(17, 32) X(18, 32)
 
 namespace asdfft {
 // True when the run-time kernel of (variant, emax) is compiled in.

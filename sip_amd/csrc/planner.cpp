@@ -117,11 +117,11 @@ std::vector<int> fitting_radices(int64_t n)
 {
     std::vector<int> r = choose_radices(n);
     if (r.empty()) return r;
-    for (int emax : {16, 32, 48}) {
+    for (int emax : {16, 32}) {
         if (threads_for(n, r, emax) > 0) return r;
     }
     for (const std::vector<int>& alt : radix_multisets(n, 3, 64)) {
-        for (int emax : {16, 32, 48}) {
+        for (int emax : {16, 32}) {
             if (threads_for(n, alt, emax) > 0) return alt;
         }
     }
@@ -164,11 +164,12 @@ bool rows_config(int64_t n, int64_t count, bool epi_lds, int want_tpb, int varia
     }
     bool found = false;
     Config best;
-    for (int emax : {16, 32, 48}) {
+    for (int emax : {16, 32}) {
         if (!has_instance(variant, emax)) continue;
         const int T = threads_for(n, radices, emax);
-        if (T == 0) continue;
-        const int maxb = max_block_for(emax);
+        // transposed stores and row pairs: 16 (32, 2) transforms in 256 / 512 threads
+        const int maxb = want_tpb <= 0 ? max_block_for(emax) : emax <= 16 ? 256 : 512;
+        if (T == 0 || T > maxb) continue;
         const int target = want_tpb > 0 ? want_tpb : std::max(1, 256 / T);
         int tpb = std::min(target, maxb / T);
         if (want_tpb <= 0) {
@@ -195,27 +196,13 @@ bool rows_config(int64_t n, int64_t count, bool epi_lds, int want_tpb, int varia
         cand.lds = lds;
         if (!found || (want_tpb > 0 && cand.tpb > best.tpb)) best = cand;
         found = true;
-        if (want_tpb <= 0) break;  // first feasible register budget (EMAX 16 preferred)
-    }
-    // Launches of one transform per workgroup and at most two per CU: where a specialised
-    // instance exists, the EMAX-16 geometry with more threads per transform (e.g. 6000 on
-    // 600 threads x 10 points instead of 200 x 30), so each CU has more waves and shorter
-    // per-thread chains to hide the latency of a single transform.  ASDFFT_WIDE_ROWS=0 turns
-    // it off.
-    const char* wr = getenv("ASDFFT_WIDE_ROWS");
-    const char* nst = getenv("ASDFFT_NO_STATIC");  // the wide geometry exists only as an instance
-    if (found && variant == kVarRowsC2C && want_tpb <= 0 && best.tpb == 1 && best.emax > 16 &&
-        count <= 2 * kNumCUs && !(wr != nullptr && wr[0] == '0') && !(nst != nullptr && nst[0] == '1')) {
-        int64_t t = 0;
-        for (int r : radices) {
-            t = (r > 16) ? 0 : std::max<int64_t>(t, (n / r + 16 / r - 1) / (16 / r));
-            if (t == 0) break;
-        }
-        if (t > 0 && t <= 1024 &&
-            find_static(kVarRowsC2C, 16, (int)n, (int)t, 0, radices.data(), (int)radices.size()) >= 0) {
-            best.emax = 16;
-            best.threads = (int)t;
-        }
+        // The first feasible register budget: 16 points per thread wherever 1024 threads hold the
+        // transform.  More threads with fewer points each give a CU more wavefronts and shorter
+        // chains, also where one workgroup fills the CU's LDS.  2^22 points a call, EMAX 32 on at
+        // most 512 threads against EMAX 16: C2C 3402 32.2 -> 19.5 us, 4320 24.0 -> 20.0, 7000 33.8
+        // -> 25.4, 10240 33.1 -> 26.7; R2C 6804 21.6 -> 16.3, C2R 12150 24.9 -> 20.3; a tenth of
+        // that many points 13 -> 9 us; 8192 and 16384 (specialised either way) 2-10% faster.
+        if (want_tpb <= 0) break;
     }
     if (found && wide8 && best.emax == 16) {
         best.threads = wide->threads;
@@ -283,28 +270,46 @@ bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_s
     // ASDFFT_COLS_LDS_CAP=<bytes> caps a column workgroup's LDS (measurement)
     const char* capenv = getenv("ASDFFT_COLS_LDS_CAP");
     const size_t lds_cap = capenv ? (size_t)atol(capenv) : kLdsLimit;
+    const char* ns = getenv("ASDFFT_NO_STATIC");
+    const bool use_static = !(ns != nullptr && ns[0] == '1');
+    // The most columns (down to 4) whose EMAX-16 workgroup lets a second one run beside it in the
+    // CU's LDS; where there is none, the most that fit at all (EMAX 16 first).  Two workgroups of
+    // up to 16 waves overlap one's loads with the other's passes: 2^22 points as X x 512, columns
+    // of 648 points 38.8 us on 16 columns at EMAX 32 (one workgroup of 6 waves per CU) -> 29.2 on 8
+    // at EMAX 16, 882 62.5 -> 31, 1500 51.6 (8) -> 38.4 (4), 324 39.3 (EMAX 32) -> 28.9.  32-byte
+    // runs of 4 columns, with neighbours on one XCD, still beat one workgroup per CU at 8; from
+    // HBM (2^24 points) the two are level.  A specialised instance of the same width goes first.
+    const auto cols_fit = [&](int tpb, int emax, size_t cap) {
+        if (!has_instance(variant, emax)) return false;
+        const int T = threads_for(n, radices, emax);
+        if (T == 0 || tpb * T > max_block_for(emax)) return false;
+        const int64_t plane = n * (tpb + 1);  // column layout: row pitch tpb + 1 words
+        const bool need_lds = radices.size() > 1 || variant == kVarColsToRows;  // (epilogue via LDS)
+        const size_t lds = need_lds ? (size_t)(8 * plane) : 0;
+        if (lds > cap || (tpb > 1 && lds > lds_cap)) return false;
+        c->radices = radices;
+        c->emax = emax;
+        c->threads = T;
+        c->tpb = (int)std::max<int64_t>(1, std::min<int64_t>(tpb, count));
+        c->tstride = 0;
+        c->plane = plane;
+        c->lds = lds;
+        return true;
+    };
     bool found = false;
-    for (int tpb : {32, 16, 8, 4, 2, 1}) {
-        if (tpb > first_tpb) continue;
-        for (int emax : {16, 32, 48}) {
-            if (!has_instance(variant, emax)) continue;
-            const int T = threads_for(n, radices, emax);
-            if (T == 0 || tpb * T > max_block_for(emax)) continue;
-            const int64_t plane = n * (tpb + 1);  // column layout: row pitch tpb + 1 words
-            const bool need_lds = radices.size() > 1 || variant == kVarColsToRows;  // (epilogue via LDS)
-            const size_t lds = need_lds ? (size_t)(8 * plane) : 0;
-            if (lds > kLdsLimit || (tpb > 1 && lds > lds_cap)) continue;
-            c->radices = radices;
-            c->emax = emax;
-            c->threads = T;
-            c->tpb = (int)std::max<int64_t>(1, std::min<int64_t>(tpb, count));
-            c->tstride = 0;
-            c->plane = plane;
-            c->lds = lds;
-            found = true;
-            break;
+    for (int tpb : {32, 16, 8, 4}) {
+        if (found || tpb > first_tpb) continue;
+        for (int emax : {16, 32}) {
+            if (found || !use_static) continue;
+            found = cols_fit(tpb, emax, kLdsLimit) && c->tpb == tpb &&
+                    find_static(variant, emax, (int)n, c->threads, tpb, radices.data(), (int)radices.size()) >= 0;
         }
-        if (found) break;
+        if (!found) found = cols_fit(tpb, 16, kLdsLimit / 2);
+    }
+    for (int tpb : {32, 16, 8, 4, 2, 1}) {
+        for (int emax : {16, 32}) {
+            if (!found && tpb <= first_tpb) found = cols_fit(tpb, emax, kLdsLimit);
+        }
     }
     // Long columns whose two LDS planes leave one workgroup per CU: a specialised kernel
     // exchanging through one plane takes the most columns (16, else 8) whose plane fits the
@@ -314,7 +319,6 @@ bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_s
     // one workgroup per CU), 83.3 us with 8 (72 KiB, two per CU) and 95.3 us on the two-plane
     // kernel (8 columns).  ASDFFT_SPLIT_EMAX=0 disables it; ASDFFT_SPLIT_EMAX / ASDFFT_SPLIT_TPB
     // force the register budget / columns per workgroup of a specialised instance (measurement).
-    const char* ns = getenv("ASDFFT_NO_STATIC");
     // ASDFFT_COLS_SPLIT=1: the one-plane kernel for every column pass that has an instance
     // (measurement)
     const char* cs = getenv("ASDFFT_COLS_SPLIT");
@@ -329,8 +333,7 @@ bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_s
     // against 81.2 us), 1024 and longer.  At 256 points (four per CU either way) the two-plane
     // kernel stays (60.4 against 62.4 us).
     const size_t four_per_cu = kLdsLimit / 4;
-    if (split_variant >= 0 && found && (c->lds > four_per_cu || prefer_split) && split_only != 0 &&
-        !(ns != nullptr && ns[0] == '1')) {
+    if (split_variant >= 0 && found && (c->lds > four_per_cu || prefer_split) && split_only != 0 && use_static) {
         bool done = false;
         for (int tpb : {16, 8}) {
             if (split_tpb_forced > 0 && tpb != split_tpb_forced) continue;
@@ -369,14 +372,17 @@ void fill_passes(const Config& c, FftArgs* a, std::vector<int>* offsets)
     }
 }
 
-// Column passes with runs shorter than a 128-byte line share lines between neighbouring
-// workgroups; keeping neighbours on one XCD lets its L2 serve the second half.
+// Column passes whose runs are not whole 128-byte lines (fewer than 16 columns, or rows that
+// do not start on a line) share lines between neighbouring workgroups; keeping neighbours on one
+// XCD lets its L2 serve the rest of the line and merge the stores to it.  384-point columns at a
+// row length of 481: 61.5 -> 56.2 us for the transform (MALL-resident, the pass 21.2 -> 16.3),
+// 236 -> 228 us from HBM; with whole lines (row length 512) level.
 // ASDFFT_XCD_REMAP=0/1 overrides (for measurement).
-int xcd_remap_for(bool cols_mapping, int tpb)
+int xcd_remap_for(bool cols_mapping, int tpb, int64_t in_stride, int64_t out_stride)
 {
     const char* e = getenv("ASDFFT_XCD_REMAP");
     if (e != nullptr && (e[0] == '0' || e[0] == '1')) return e[0] - '0';
-    return (cols_mapping && tpb < 16) ? 1 : 0;
+    return (cols_mapping && (tpb < 16 || in_stride % 16 != 0 || out_stride % 16 != 0)) ? 1 : 0;
 }
 
 // Row launches of at most this many workgroups take a twiddle-preloading instance where one
@@ -456,7 +462,7 @@ bool stockham_step(int64_t n, int variant, bool cols_mapping, const StepIo& io, 
     a.out_inner = io.out_inner;
     a.out_outer = io.out_outer;
     a.out_stride = io.out_stride;
-    a.xcd_remap = xcd_remap_for(cols_mapping, c.tpb);
+    a.xcd_remap = xcd_remap_for(cols_mapping, c.tpb, io.in_stride, io.out_stride);
     a.in_o_mod = 1;
     a.out_scale = 1.0f;
     a.o_split = io.o_split;
@@ -1019,7 +1025,8 @@ bool mfma_fourstep(int64_t n, int64_t count, bool inverse, BuiltPlan* bp, std::s
 
 }  // namespace
 
-int max_block_for(int emax) { return emax <= 16 ? 256 : 512; }
+// Run-time kernels of both register budgets are bounded at 1024 threads.
+int max_block_for(int) { return 1024; }
 
 namespace {
 

@@ -814,11 +814,17 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
     }
 }
 
+// Workgroup of the specialised row kernels that keep their transforms per workgroup at run time.
 template <int EMAX>
 constexpr int max_block()
 {
     return EMAX <= 16 ? 256 : 512;
 }
+
+// Largest workgroup of the run-time kernels.  1024 threads allow 128 VGPRs; the EMAX-16 kernels
+// take 63 to 78 and the EMAX-32 ones 95 to 104, so the bound costs no registers, and a transform
+// or a column tile can have twice to four times the wavefronts per CU that 256 / 512 threads gave.
+constexpr int kRuntimeBlock = 1024;
 
 // Occupancy target of kernels that run EMAX-16 transforms in 512-thread workgroups: at
 // most 128 VGPRs (4 waves per SIMD); EMAX-32 kernels hold twice the points.
@@ -831,7 +837,7 @@ constexpr int min_waves()
 
 // ------------------------------------------------------------------ runtime kernel
 template <int EMAX, int MAP, int PRO, int EPI>
-__global__ void __launch_bounds__(max_block<EMAX>()) stockham_kernel(const FftArgs a)
+__global__ void __launch_bounds__(kRuntimeBlock) stockham_kernel(const FftArgs a)
 {
     extern __shared__ float smem[];
     float* lre = smem;
