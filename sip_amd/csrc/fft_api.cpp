@@ -40,6 +40,8 @@ enum class PlanState { kCreated, kInitialized, kFailed };
 // time and the overlap-add geometry.
 struct IstftDesc {
     int64_t channel = 0, nfft = 0, nframes = 0, hop = 0, win_length = 0, out_len = 0;
+    bool fused = false;              // one launch (fused_plan); else frames into the workspace, then overlap-add
+    asdfft::IstftFusedPlan fused_plan;
 };
 
 struct FftPlan {
@@ -830,6 +832,8 @@ AspbStatus asdFftIstftMakePlan(asdFftHandle handle, const aclTensor* input, cons
         log_error(fn, why);
         return ACL_ERROR_INTERNAL_ERROR;
     }
+    d.fused = asdfft::build_istft_fused(built, d.nfft, d.channel, d.nframes, d.hop, &d.fused_plan);
+    if (d.fused) built.steps[0].describe += "; run as " + d.fused_plan.describe;
     p.type = ASCEND_FFT_C2C;
     p.direction = ASCEND_FFT_INVERSE;
     p.sizes = {nFft};
@@ -905,9 +909,11 @@ AspbStatus asdFftExecIstft(asdFftHandle handle, const aclTensor* input, const ac
     const AspbStatus dev = check_device(p.built, fn);
     if (dev != ACL_SUCCESS) return dev;
     hipStream_t stream = static_cast<hipStream_t>(p.stream);
-    char* bufs[3] = {in, out, static_cast<char*>(p.workspace)};
-    const AspbStatus st = launch_steps(p.built, bufs, nullptr, nullptr, stream, fn, -1);
-    if (st != ACL_SUCCESS) return st;
+    if (!d->fused) {
+        char* bufs[3] = {in, out, static_cast<char*>(p.workspace)};
+        const AspbStatus st = launch_steps(p.built, bufs, nullptr, nullptr, stream, fn, -1);
+        if (st != ACL_SUCCESS) return st;
+    }
     asdfft::OlaArgs a{};
     a.frames = p.workspace;
     a.window = reinterpret_cast<const float*>(win);
@@ -919,7 +925,15 @@ AspbStatus asdFftExecIstft(asdFftHandle handle, const aclTensor* input, const ac
     a.channel = d->channel;
     a.out_len = d->out_len;
     a.scale = 1.0f / (float)d->nfft;
-    const hipError_t e = asdfft::launch_istft_ola(a, stream);
+    hipError_t e;
+    if (d->fused) {
+        asdfft::IstftFusedArgs f = d->fused_plan.args;
+        f.ola = a;
+        f.spec = in;
+        e = asdfft::launch_istft_fused(f, d->fused_plan.grid, d->fused_plan.lds_bytes, stream);
+    } else {
+        e = asdfft::launch_istft_ola(a, stream);
+    }
     if (e != hipSuccess) {
         log_error(fn, std::string("kernel launch failed: ") + hipGetErrorString(e));
         return ACL_ERROR_INTERNAL_ERROR;

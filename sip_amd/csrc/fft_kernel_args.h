@@ -178,4 +178,17 @@ struct OlaArgs {
     float scale;         // 1 / nfft
 };
 
+// ISTFT in one launch (istft_fused.hip): a workgroup transforms frames in groups of fft.tpb and
+// makes chunk_frames * hop samples of one channel.
+struct IstftFusedArgs {
+    FftArgs fft;           // n, threads, tpb, passes and twiddles of the frame transform
+    OlaArgs ola;           // frames unused
+    const void* spec;      // complex [channel][nfft][nframes]
+    int groups;            // groups a workgroup walks
+    int halo;              // frames before the chunk that reach its samples: ceil(nfft / hop) - 1
+    uint32_t hop_magic;    // floor(2^32 / hop) + 1
+    int64_t chunk_frames;  // groups * fft.tpb - halo
+    int64_t chunks;        // workgroups per channel
+};
+
 }  // namespace asdfft

@@ -91,6 +91,8 @@ int dft_pairs_per_block();
 hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, hipStream_t stream);
 // Radices of the first / second transform of convolution length m (empty: no kernel).
 std::vector<int> bluestein_radices(int64_t m, bool second);
+bool istft_fused_radix(int radix);  // radix compiled into istft_fused_kernel
+hipError_t launch_istft_fused(const IstftFusedArgs& args, int64_t grid, size_t lds_bytes, hipStream_t stream);
 hipError_t launch_istft_ola(const OlaArgs& args, hipStream_t stream);
 hipError_t launch_real_aux(const RealAuxArgs& args, hipStream_t stream);
 

@@ -1594,6 +1594,71 @@ std::string build_istft_frames(int64_t nfft, int64_t channel, int64_t nframes, B
     return "";
 }
 
+// Where one launch can do: frame lengths whose passes fit 16 points per thread, at most F + 1
+// frames over a sample.  Of the frames per group (16 = 128-byte runs of the spectrum, 8, 4) and
+// the groups per workgroup, the pair of least time: launch rounds x (groups + 1/2) x (what the
+// workgroups of one CU compute per group, about 0.75 us per 1024 points, + 5 us of latency).
+// Separate launches -> one, us: 16 x 1024 x 1000 frames, hop 256 122 -> 84; 16 x 512 x 1000, hop 128
+// 67 -> 41; 12 x 720 x 500, hop 180 49 -> 32; 16 x 128 x 1000, hop 32 23 -> 12; 1 x 128 x 50 14.6 -> 11.
+bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, int64_t nframes, int64_t hop,
+                       IstftFusedPlan* out)
+{
+    if (frames.steps.size() != 1 || frames.steps[0].direct || frames.steps[0].shape.emax != 16) return false;
+    const FftArgs& step = frames.steps[0].args;
+    std::vector<int> radices;
+    for (int p = 0; p < step.passes; p++) {
+        if (!istft_fused_radix(step.pass[p].radix)) return false;
+        radices.push_back(step.pass[p].radix);
+    }
+    const int T = threads_for(nfft, radices, 16);
+    const int64_t reach = (nfft + hop - 1) / hop;  // frames that reach one sample
+    const PassDesc& last = step.pass[step.passes - 1];
+    const int64_t twiddles = step.passes > 1 ? last.tw_offset + (int64_t)last.span * (last.radix - 1) : 0;
+    IstftFusedPlan best;
+    double cost = 1e300;
+    for (int F : {16, 8, 4}) {
+        // the carry holds what one later group adds to: its samples are done before the next
+        if (T == 0 || T * F > max_block_for(16) || hop > nfft || hop * (F + 1) < nfft) continue;
+        const size_t lds = (size_t)(nfft * (F + 1) + nfft - hop + twiddles) * 8 + (size_t)(nfft + hop) * 4;
+        if (lds > kLdsLimit) continue;
+        // 128 VGPRs: 16 waves per CU
+        const int64_t per_cu = std::min<int64_t>(16 / ((T * F + 63) / 64), (int64_t)(kLdsLimit / lds));
+        const int64_t span = nframes + reach - 1;  // hops that hold samples
+        for (int64_t groups = 1; groups <= 4096; groups++) {
+            const int64_t chunk = groups * F - (reach - 1);
+            if (chunk <= 0) continue;
+            const int64_t chunks = (span + chunk - 1) / chunk;
+            const int64_t grid = channel * chunks;
+            const int64_t rounds = (grid + per_cu * kNumCUs - 1) / (per_cu * kNumCUs);
+            const int64_t beside = std::min<int64_t>(per_cu, (grid + kNumCUs - 1) / kNumCUs);
+            const double c = (double)rounds * ((double)groups + 0.5) *
+                             (0.75 * (double)(beside * F) * (double)nfft / 1024.0 + 5.0);
+            if (c < cost && grid <= 0x7fffffff) {
+                cost = c;
+                best.args.groups = (int)groups;
+                best.args.chunk_frames = chunk;
+                best.args.chunks = chunks;
+                best.grid = grid;
+                best.lds_bytes = lds;
+                best.args.fft = step;
+                best.args.fft.tpb = F;
+                best.args.fft.threads = T;
+            }
+            if (chunks == 1) break;
+        }
+    }
+    if (best.grid == 0) return false;
+    best.args.halo = (int)(reach - 1);
+    best.args.hop_magic = (uint32_t)(((uint64_t)1 << 32) / (uint64_t)hop + 1);
+    std::ostringstream os;
+    os << "istft fused frames/group=" << best.args.fft.tpb << " T=" << T << " groups=" << best.args.groups
+       << " halo=" << best.args.halo << " chunks=" << best.args.chunks << " lds=" << best.lds_bytes
+       << " grid=" << best.grid;
+    best.describe = os.str();
+    *out = best;
+    return true;
+}
+
 hipError_t launch_step(const Step& s, char* const bufs[3], const float* in_im, float* out_im, hipStream_t stream)
 {
     if (s.mfma) {

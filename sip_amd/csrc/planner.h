@@ -120,6 +120,17 @@ std::string build_plan(const PlanSpec& spec, BuiltPlan* out);
 // dst kBufWork).  Returns "" on success, otherwise the reason.
 std::string build_istft_frames(int64_t nfft, int64_t channel, int64_t nframes, BuiltPlan* out);
 
+// Geometry of the one-launch ISTFT (istft_fused.hip) for a plan whose frame transforms are
+// `frames`; false where the two launches stay.  spec, window and out are filled per call.
+struct IstftFusedPlan {
+    IstftFusedArgs args{};
+    int64_t grid = 0;
+    size_t lds_bytes = 0;
+    std::string describe;
+};
+bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, int64_t nframes, int64_t hop,
+                       IstftFusedPlan* out);
+
 // Launch of one step on `stream`: bufs = {input, output, workspace}; planar steps take the
 // imaginary planes from in_im / out_im.
 hipError_t launch_step(const Step& s, char* const bufs[3], const float* in_im, float* out_im, hipStream_t stream);

@@ -117,3 +117,33 @@ def test_istft_inverts_a_gpu_stft(torch_dev):
     ref = sig[:, :out.shape[1]]
     err = (torch.linalg.vector_norm(out - ref) / torch.linalg.vector_norm(ref)).item()
     assert err < 1e-5, err
+
+
+# one launch (istft_fused.hip): frames over a sample up to and past what a group holds (128: hop 8,
+# 7), one-pass frames, one frame, hop = nfft, a single group and many per workgroup, frames that
+# leave the last group nearly empty, channels enough for several rounds, the widest frames
+FUSED = [(2, 128, 70, 8), (1, 128, 40, 7), (3, 16, 33, 4), (2, 12, 17, 12), (600, 64, 70, 16),
+         (40, 1024, 65, 512), (70, 420, 49, 140), (5, 1440, 21, 360), (3, 1000, 18, 999)]
+
+
+@pytest.mark.parametrize("channel,nfft,nframes,hop", FUSED, ids=str)
+def test_istft_one_launch(torch_dev, oracle, channel, nfft, nframes, hop):
+    import torch
+
+    from oracle.oracle import rel_l2_per_row
+    from sip_amd import Istft
+    rng = np.random.default_rng(nfft + nframes)
+    spec = (rng.uniform(-1, 1, (channel, nfft, nframes)) +
+            1j * rng.uniform(-1, 1, (channel, nfft, nframes))).astype(np.complex64)
+    w = window(nfft)
+    p = Istft(channel, nfft, nframes, hop)
+    try:
+        assert ("istft fused" in p.describe()) == ((nfft, hop) != (128, 7)), p.describe()
+        out = torch.full((channel, p.out_len), float("nan"), dtype=torch.complex64, device=torch_dev)
+        if p.out_len == 0:
+            return
+        p.execute(torch.from_numpy(spec).to(torch_dev), torch.from_numpy(w).to(torch_dev), out=out)
+        got = out.cpu().numpy()
+    finally:
+        p.close()
+    assert rel_l2_per_row(got, oracle.istft(spec, w, hop), 1).max() <= tol_for(nfft)
