@@ -42,7 +42,7 @@ KERNEL_HEADERS = ["stockham_impl.h", "fft_kernel_args.h", "kernels.h", "radix_co
 KERNEL_SOURCES = ["dft_direct.hip", "bluestein.hip", "mfma_fft.hip", "shift_kernel.hip", "istft_kernel.hip", "istft_fused.hip", "real_aux.hip",
                   "static_scratch.hip", "wave_fft.hip"]
 # the ragged kernel builds once per register budget (one translation unit each)
-RAGGED_EMAX = [16, 32, 48]
+RAGGED_EMAX = [16, 20, 24, 32, 48]
 
 
 def instances():

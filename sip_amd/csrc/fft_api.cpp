@@ -1183,7 +1183,10 @@ extern "C" int32_t asdFftExtMakePlanRagged(void* handle, const asdFftExtRaggedEn
     // transform) in a launch of their own beside the single launch of the others (measured
     // within 3% of the single launch: 100.6 vs 103.3 us on the 4000-transform workload)
     opt.wide16 = false;
-    if (const char* w = getenv("ASDFFT_RAGGED_WIDE16")) opt.wide16 = opt.one_launch && w[0] == '1';
+    if (const char* w = getenv("ASDFFT_RAGGED_WIDE16")) {
+        opt.wide16 = opt.one_launch && w[0] == '1';
+        opt.sized = false;
+    }
     auto plan = std::make_unique<asdfft::RaggedPlan>();
     bool unsupported = false;
     std::string why;

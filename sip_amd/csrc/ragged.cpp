@@ -22,7 +22,9 @@ namespace asdfft {
 
 namespace {
 
-constexpr size_t kLdsLimit = kRaggedLdsLimit;
+// Most LDS a workgroup of a budget takes.
+size_t ragged_lds_for(int emax) { return emax == kRaggedHalf ? kRaggedHalfLds : kRaggedLdsLimit; }
+
 constexpr size_t kLdsFloor = 64 * 1024;
 constexpr int64_t kMaxComplexLength = 16384;  // one class's transform fits one workgroup's LDS
 
@@ -74,6 +76,48 @@ size_t class_lds(const RaggedClassInfo& c, int tpb)
     return need_lds(c) ? (size_t)8 * (size_t)tpb * (size_t)(pad16(c.n) + 1) : 0;
 }
 
+// Schedule of a class in the launch of budget kRaggedHalf or kRaggedWide: the fewest-pass radices that
+// fit (a fixed schedule's otherwise), on 16 points per thread or the budget's, whichever fills a tile
+// with more points.  False where nothing fits.
+bool sized_schedule(RaggedClassInfo* cp, const ClassSchedule* fixed, int emax)
+{
+    const int block = ragged_block_for(emax);
+    const size_t lds = ragged_lds_for(emax);
+    std::vector<std::vector<int>> sets;
+    if (fixed != nullptr) {
+        sets.push_back(fixed->radices);
+    } else {
+        sets = radix_multisets(cp->n, 3, 64);
+        sets.insert(sets.begin(), choose_radices(cp->n));
+    }
+    for (const std::vector<int>& radices : sets) {
+        int64_t prod = 1;
+        for (int r : radices) prod *= r;
+        if (prod != cp->n || radices.empty() || (int)radices.size() > kMaxPasses) return false;
+        int64_t most = 0;
+        for (int e : {16, emax}) {
+            RaggedClassInfo c = *cp;
+            c.emax = emax;
+            c.sched.radices = radices;
+            c.sched.threads = min_threads(c.n, radices, e);
+            c.sched.tpb = 0;
+            if (fixed != nullptr) {
+                c.sched.threads = c.sched.threads > 0 ? std::max(c.sched.threads, fixed->threads) : 0;
+                c.sched.tpb = fixed->tpb;
+            }
+            if (c.sched.threads == 0 || c.sched.threads > block || class_lds(c, 1) > lds) continue;
+            int tpb = block / c.sched.threads;
+            while (tpb > 1 && class_lds(c, tpb) > lds) tpb--;
+            if (tpb * c.n > most) {
+                most = tpb * c.n;
+                *cp = c;
+            }
+        }
+        if (most > 0) return true;
+    }
+    return false;
+}
+
 int device_cus()
 {
     int dev = 0, n = 0;
@@ -91,7 +135,7 @@ void free_device(void* p)
 
 }  // namespace
 
-int ragged_block_for(int emax) { return emax <= 16 ? 256 : 512; }
+int ragged_block_for(int emax) { return emax <= 16 ? 256 : emax == kRaggedWide ? kRaggedMaxBlock16 : 512; }
 
 // ---- dispatch over the per-budget kernel translation units
 #define ASDFFT_RAGGED_DECL(E)                                                                        \
@@ -100,28 +144,32 @@ int ragged_block_for(int emax) { return emax <= 16 ? 256 : 512; }
     hipError_t launch_ragged_e##E(int64_t grid, int block, size_t lds_bytes, const RaggedArgs& args, \
                                   const RaggedClass* classes, const RaggedTile* tiles, hipStream_t stream);
 ASDFFT_RAGGED_DECL(16)
+ASDFFT_RAGGED_DECL(20)
+ASDFFT_RAGGED_DECL(24)
 ASDFFT_RAGGED_DECL(32)
 ASDFFT_RAGGED_DECL(48)
 #undef ASDFFT_RAGGED_DECL
+#define ASDFFT_RAGGED_BY_EMAX(FN, ARGS) \
+    if (emax <= 16) return FN##_e16 ARGS; \
+    if (emax <= 20) return FN##_e20 ARGS; \
+    if (emax <= 24) return FN##_e24 ARGS; \
+    if (emax <= 32) return FN##_e32 ARGS; \
+    return FN##_e48 ARGS;
 
 const void* ragged_kernel_fn(int emax)
 {
-    if (emax <= 16) return ragged_kernel_fn_e16();
-    return emax <= 32 ? ragged_kernel_fn_e32() : ragged_kernel_fn_e48();
+    ASDFFT_RAGGED_BY_EMAX(ragged_kernel_fn, ())
 }
 
 hipError_t ragged_prepare(int emax, size_t lds_bytes, int block, int* per_cu)
 {
-    if (emax <= 16) return ragged_prepare_e16(lds_bytes, block, per_cu);
-    return emax <= 32 ? ragged_prepare_e32(lds_bytes, block, per_cu) : ragged_prepare_e48(lds_bytes, block, per_cu);
+    ASDFFT_RAGGED_BY_EMAX(ragged_prepare, (lds_bytes, block, per_cu))
 }
 
 hipError_t launch_ragged(int emax, int64_t grid, int block, size_t lds_bytes, const RaggedArgs& args,
                          const RaggedClass* classes, const RaggedTile* tiles, hipStream_t stream)
 {
-    if (emax <= 16) return launch_ragged_e16(grid, block, lds_bytes, args, classes, tiles, stream);
-    if (emax <= 32) return launch_ragged_e32(grid, block, lds_bytes, args, classes, tiles, stream);
-    return launch_ragged_e48(grid, block, lds_bytes, args, classes, tiles, stream);
+    ASDFFT_RAGGED_BY_EMAX(launch_ragged, (grid, block, lds_bytes, args, classes, tiles, stream))
 }
 
 int64_t ragged_in_bytes(const RaggedEntry& e)
@@ -297,6 +345,45 @@ RaggedPlan::~RaggedPlan()
 
 namespace {
 
+// Geometry of the single launch.  A workgroup's phases (load, exchanges, store) follow one another, so
+// what a CU gets done is set by how many wavefronts it holds and into how many workgroups they are
+// split.  The batches of mixed lengths, 70% C2C and 30% R2C, log-uniform over 64..nmax:
+//   * every class within the EMAX-16 budget (256 threads): left to it, four workgroups per CU;
+//   * every class within half a CU's LDS (about 9600 points): 512 threads of up to 24 points, two
+//     workgroups of 8 wavefronts per CU.  4000 transforms to 8192 50.1 -> 43.9 us, 2000 to 8192
+//     30.3 -> 25.8, 4000 to 4096 29.0 -> 27.2 against 32 points per thread, one workgroup per CU;
+//   * else every class on 1024 threads of up to 20 points, one workgroup of 16 wavefronts per CU
+//     (128 VGPRs): 4000 transforms to 16384 101.7 -> 84.2 us, 1000 33.4 -> 29.2, 300 26.4 -> 22.2
+//     against 48 points on 512 threads.  The short classes in a launch of their own at half a CU
+//     take 90 us, after the long ones or beside them: the long tiles' last round is nearly empty;
+//   * false where a class fits neither (13, 17, 19 in lengths near 16384): one launch at the largest
+//     register budget, as before.
+bool single_launch_geometry(const RaggedOptions& opt, std::vector<RaggedClassInfo>* classes)
+{
+    bool fits16 = true;
+    for (const RaggedClassInfo& c : *classes) {
+        auto f = opt.fixed.find(c.key);
+        RaggedClassInfo own = c;
+        bool unsupported = false;
+        fits16 = fits16 && ragged_schedule(&own, f != opt.fixed.end() ? &f->second : nullptr, &unsupported).empty() &&
+                 own.emax <= 16;
+    }
+    if (fits16) return false;
+    for (int emax : {kRaggedHalf, kRaggedWide}) {
+        std::vector<RaggedClassInfo> sized = *classes;
+        bool fits = true;
+        for (RaggedClassInfo& c : sized) {
+            auto f = opt.fixed.find(c.key);
+            fits = fits && sized_schedule(&c, f != opt.fixed.end() ? &f->second : nullptr, emax);
+        }
+        if (fits) {
+            *classes = sized;
+            return true;
+        }
+    }
+    return false;
+}
+
 std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOptions& opt, RaggedPlan* plan,
                        bool* unsupported)
 {
@@ -362,7 +449,8 @@ std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOpti
     plan->all_inplace_c2c = inplace;
 
     // ---- per-class schedules
-    for (size_t ci = 0; ci < plan->classes.size(); ci++) {
+    const bool sized = opt.one_launch && !opt.wide16 && opt.sized && single_launch_geometry(opt, &plan->classes);
+    for (size_t ci = 0; ci < plan->classes.size() && !sized; ci++) {
         RaggedClassInfo& c = plan->classes[ci];
         auto f = opt.fixed.find(c.key);
         const std::string why = ragged_schedule(&c, f != opt.fixed.end() ? &f->second : nullptr, unsupported,
@@ -370,12 +458,12 @@ std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOpti
         if (!why.empty()) return why;
     }
 
-    // one launch for the whole batch: every class takes the largest register budget (a
+    // otherwise one launch for the whole batch: every class takes the largest register budget (a
     // class keeps its thread count; the extra butterfly slots of a larger budget stay idle).
     // With wide EMAX-16 schedules (up to 1024 threads per transform, more than the larger
     // budgets' 512-thread workgroups hold) the EMAX-16 classes keep a launch of their own and
     // only the others share the largest budget: two launches at most.
-    if (opt.one_launch) {
+    if (opt.one_launch && !sized) {
         int top = 0, top_rest = 0;
         for (const RaggedClassInfo& c : plan->classes) {
             top = std::max(top, c.emax);
@@ -391,7 +479,7 @@ std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOpti
     }
 
     // ---- launches: one per register budget
-    for (int emax : {16, 32, 48}) {
+    for (int emax : {16, kRaggedWide, kRaggedHalf, 32, 48}) {
         RaggedLaunchPlan L;
         L.emax = emax;
         int maxT = 0;
@@ -409,7 +497,8 @@ std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOpti
         block = std::min(block, ragged_max_block(emax));
         L.block = block;
         // whole workgroups of transforms: tiles fill every lane that LDS allows
-        const size_t budget = std::min(kLdsLimit, std::max(kLdsFloor, one * (size_t)std::max(1, block / maxT)));
+        const size_t floor = emax == kRaggedHalf ? kRaggedHalfLds : kLdsFloor;
+        const size_t budget = std::min(ragged_lds_for(emax), std::max(floor, one * (size_t)std::max(1, block / maxT)));
         for (int ci : L.class_ids) {
             RaggedClassInfo& c = plan->classes[ci];
             if (c.sched.threads > block) {  // every transform of a tile needs its threads in the workgroup

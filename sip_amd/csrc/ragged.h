@@ -18,11 +18,16 @@
 
 namespace asdfft {
 
-// Largest workgroup of the ragged kernel (its __launch_bounds__): 1024 threads for the EMAX-16
-// kernel (at most 128 VGPRs, which that budget meets), 512 for the EMAX-32 and EMAX-48 ones.
+// Largest workgroup of the ragged kernel (its __launch_bounds__): 1024 threads for the EMAX-16 and
+// EMAX-20 kernels (at most 128 VGPRs; they take 95), 512 for the larger budgets.
 constexpr int kRaggedMaxBlock = 512;
 constexpr int kRaggedMaxBlock16 = 1024;
-constexpr int ragged_max_block(int emax) { return emax <= 16 ? kRaggedMaxBlock16 : kRaggedMaxBlock; }
+constexpr int ragged_max_block(int emax) { return emax <= 20 ? kRaggedMaxBlock16 : kRaggedMaxBlock; }
+// Budgets of a single launch: 512 threads of up to 24 points in at most half a CU's LDS, and 1024
+// threads of up to 20 (5^6 fits 20 points and not 16).
+constexpr int kRaggedHalf = 24;
+constexpr int kRaggedWide = 20;
+constexpr size_t kRaggedHalfLds = 80 * 1024;
 // Dynamic LDS a ragged launch may take: the workgroup's 160 KiB less room for the
 // kernel's static tile index.
 constexpr size_t kRaggedLdsLimit = 160 * 1024 - 256;
@@ -58,6 +63,7 @@ struct RaggedOptions {
     bool autotune = false;  // time candidate schedules on the device at plan time
     bool one_launch = true;  // every class in one launch at the largest register budget (false:
                              // one concurrent launch per register budget)
+    bool sized = true;       // one launch: its geometry by the longest class (single_launch_geometry)
     bool wide16 = false;     // EMAX-16 schedules of up to 1024 threads per transform before larger budgets
                              // (the EMAX-16 classes then take a launch of their own: two launches)
     int block16 = 0;        // workgroup size of the EMAX-16 launch (0: automatic)

@@ -121,7 +121,7 @@ ragged_kernel(const RaggedArgs r, const RaggedClass* __restrict__ classes, const
 }  // namespace
 
 // Entry points of this translation unit's register budget (the build compiles this file
-// once per EMAX in {16, 32, 48}; ragged.cpp dispatches on the budget).
+// once per EMAX in {16, 20, 24, 32, 48}; ragged.cpp dispatches on the budget).
 #ifndef ASDFFT_RAGGED_EMAX
 #error "ASDFFT_RAGGED_EMAX must be defined"
 #endif

@@ -831,7 +831,7 @@ constexpr int kRuntimeBlock = 1024;
 template <int EMAX>
 constexpr int min_waves()
 {
-    return EMAX <= 16 ? 4 : 1;
+    return EMAX <= 24 ? 4 : 1;
 }
 
 
