@@ -12,6 +12,7 @@ import os
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libasdfft.so")
 TORCH_LIB_PATH = os.path.join(HERE, "lib", "libasdfft_torch.so")
+PY_EXEC_PATH = os.path.join(HERE, "lib", "_asdfft_py.so")
 
 # asdFftType / asdFftDirection / asdFft1dDimType (include/fft_api.h)
 ASCEND_FFT_C2C = 0x10
@@ -198,6 +199,27 @@ def torch_ops():
         torch.ops.load_library(TORCH_LIB_PATH)
         _torch_ops = torch.ops.torch_sip
     return _torch_ops
+
+
+_py_exec = None
+
+
+def py_exec():
+    """Load the extension module _asdfft_py once; raises NativeLibraryMissing if it has not been built."""
+    global _py_exec
+    if _py_exec is None:
+        import importlib.machinery
+        import importlib.util
+
+        import torch  # noqa: F401  (the module links against torch's libraries)
+        if not os.path.exists(PY_EXEC_PATH):
+            raise NativeLibraryMissing(f"{PY_EXEC_PATH} not built; run `python -m sip_amd.build`")
+        lib()
+        loader = importlib.machinery.ExtensionFileLoader("_asdfft_py", PY_EXEC_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_asdfft_py", loader))
+        loader.exec_module(module)
+        _py_exec = module
+    return _py_exec
 
 
 def check(fn: str, status: int) -> None:

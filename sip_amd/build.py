@@ -22,7 +22,6 @@ INCLUDE = os.path.join(ROOT, "include")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libasdfft.so")
-TORCH_LIB = os.path.join(LIBDIR, "libasdfft_torch.so")
 ARCH = os.environ.get("ASDFFT_ARCH", "gfx950")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
@@ -120,23 +119,37 @@ def _run(cmd):
     return out
 
 
-def build_torch_ops(force: bool = False) -> str:
-    """libasdfft_torch.so: the torch_sip operators (torch_ops.cpp) over libasdfft.so."""
+def _build_torch_library(name: str, source: str, force: bool, python: bool) -> str:
+    import sysconfig
+
     import torch
     tdir = os.path.dirname(torch.__file__)
-    src = os.path.join(CSRC, "torch_ops.cpp")
+    src, out = os.path.join(CSRC, source), os.path.join(LIBDIR, name)
     deps = [src, LIB] + [os.path.join(INCLUDE, h) for h in os.listdir(INCLUDE) if h.endswith(".h")]
-    if not force and not _newer(TORCH_LIB, deps):
-        return TORCH_LIB
+    if not force and not _newer(out, deps):
+        return out
     abi = int(torch.compiled_with_cxx11_abi())
-    tmp = TORCH_LIB + ".tmp"
+    tmp = out + ".tmp"
+    py = [f"-I{sysconfig.get_path('include')}"] if python else []
+    # the interpreter itself provides the Python symbols of an extension module
+    end = ["-ltorch_python"] if python else ["-Wl,--no-undefined"]
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DUSE_ROCM",
-          "-D__HIP_PLATFORM_AMD__", f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include",
-          f"-I{ROCM}/include", f"-I{INCLUDE}", src, "-o", tmp, f"-L{tdir}/lib", "-lc10", "-lc10_hip", "-ltorch",
+          "-D__HIP_PLATFORM_AMD__", f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include"] + py +
+         [f"-I{ROCM}/include", f"-I{INCLUDE}", src, "-o", tmp, f"-L{tdir}/lib", "-lc10", "-lc10_hip", "-ltorch",
           "-ltorch_cpu", "-ltorch_hip", f"-L{LIBDIR}", "-lasdfft", f"-L{ROCM}/lib", "-lamdhip64",
-          "-Wl,-rpath,$ORIGIN", "-Wl,--no-undefined"])
-    os.replace(tmp, TORCH_LIB)
-    return TORCH_LIB
+          "-Wl,-rpath,$ORIGIN"] + end)
+    os.replace(tmp, out)
+    return out
+
+
+def build_torch_ops(force: bool = False) -> str:
+    """libasdfft_torch.so: the torch_sip operators (torch_ops.cpp) over libasdfft.so."""
+    return _build_torch_library("libasdfft_torch.so", "torch_ops.cpp", force, python=False)
+
+
+def build_py_exec(force: bool = False) -> str:
+    """_asdfft_py.so: the extension module behind Plan.execute and Istft.execute (py_exec.cpp)."""
+    return _build_torch_library("_asdfft_py.so", "py_exec.cpp", force, python=True)
 
 
 def host_driver(driver: str, out: str, sanitize: str | None = None, jobs: int | None = None) -> str:
@@ -230,6 +243,7 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = False) -
              [f"-L{ROCM}/lib", "-lamdhip64", "-Wl,--no-undefined"])
         os.replace(tmp, LIB)
     build_torch_ops(force)
+    build_py_exec(force)
     return LIB
 
 

@@ -67,7 +67,7 @@ class Plan:
             self.handle = None
             raise
         self._workspace = None
-        self._stream = None
+        self._code = t
 
     # --- shapes -------------------------------------------------------------------------
     def in_shape(self):
@@ -101,29 +101,38 @@ class Plan:
         return [arr[i] for i in range(n.value)]
 
     # --- execution (torch device tensors) ---------------------------------------------------
-    def bind_workspace(self, device):
-        import torch
+    def workspace_on(self, device):
         if self.workspace_size and (self._workspace is None or self._workspace.device != device):
+            import torch
             self._workspace = torch.empty(self.workspace_size, dtype=torch.uint8, device=device)
+        return self._workspace
+
+    def bind_workspace(self, device):
+        self.workspace_on(device)
         if self.workspace_size:
             N.check("asdFftSetWorkspace", self.L.asdFftSetWorkspace(self.handle, self._workspace.data_ptr()))
 
     def bind_stream(self, stream_handle: int):
         # torch's default stream is the null stream, refused by asdFftSetStream; hipStreamLegacy
         # ((hipStream_t)1) names that same stream
-        stream_handle = stream_handle or 1
-        if stream_handle != self._stream:
-            N.check("asdFftSetStream", self.L.asdFftSetStream(self.handle, ctypes.c_void_p(stream_handle)))
-            self._stream = stream_handle
+        N.check("asdFftSetStream", self.L.asdFftSetStream(self.handle, ctypes.c_void_p(stream_handle or 1)))
 
     def execute(self, x, out=None):
         """Runs the plan on torch device tensor x (complex64 or float32); returns out."""
-        import torch
         if self.kind == "c2c_sep":
             raise TypeError("a c2c_sep plan runs through execute_separated")
         if out is None:
+            import torch
             dt = torch.float32 if self.kind == "c2r" else torch.complex64
             out = torch.empty(self.out_shape(), dtype=dt, device=x.device)
+        if self.handle is not None:
+            ws = self.workspace_on(x.device) if self.workspace_size else None
+            bad = N.py_exec().execute(self.handle.value, self._code, ws, x, out)
+            if bad is None:
+                return out
+            if bad is not NotImplemented:
+                N.check(*bad)
+        import torch
         self.bind_workspace(x.device)
         self.bind_stream(torch.cuda.current_stream(x.device).cuda_stream)
         xin = N.AclTensor(x.shape, N.ACL_FLOAT if x.dtype == torch.float32 else N.ACL_COMPLEX64, x.data_ptr())
@@ -198,7 +207,6 @@ class Istft:
         finally:
             shape.close()
         self._workspace = None
-        self._stream = None
 
     def describe(self) -> str:
         need = ctypes.c_size_t(0)
@@ -207,14 +215,23 @@ class Istft:
         self.L.asdFftExtDescribePlan(self.handle, buf, len(buf), None)
         return buf.value.decode()
 
+    workspace_on = Plan.workspace_on
     bind_workspace = Plan.bind_workspace
     bind_stream = Plan.bind_stream
 
     def execute(self, spec, window, out=None):
         """spec: complex64 (channel, nfft, nframes) device tensor; window: float32 (nfft,)."""
-        import torch
         if out is None:
+            import torch
             out = torch.empty((self.channel, self.out_len), dtype=torch.complex64, device=spec.device)
+        if self.handle is not None:
+            ws = self.workspace_on(spec.device) if self.workspace_size else None
+            bad = N.py_exec().execute_istft(self.handle.value, ws, spec, window, out)
+            if bad is None:
+                return out
+            if bad is not NotImplemented:
+                N.check(*bad)
+        import torch
         self.bind_workspace(spec.device)
         self.bind_stream(torch.cuda.current_stream(spec.device).cuda_stream)
         ts = [N.AclTensor(t.shape, N.ACL_FLOAT if t.dtype == torch.float32 else N.ACL_COMPLEX64, t.data_ptr())
