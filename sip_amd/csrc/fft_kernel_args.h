@@ -55,6 +55,7 @@ struct PassDesc {
     int span;         // L: product of the radices of the earlier passes
     uint32_t magic;   // floor(2^32 / L) + 1 (L > 1): j / L == umulhi(j, magic)
     int tw_offset;    // first entry of this pass in the twiddle table (layout [k][r-1])
+    int read_step;    // ragged kernels: LDS points between a butterfly's inputs (N / R, more where padded)
 };
 
 struct FftArgs {
@@ -71,6 +72,7 @@ struct FftArgs {
     int tpb;                // transforms per workgroup
     int passes;
     int lds_tstride;        // row mapping: padded LDS words per transform
+    int lds_pad;            // ragged kernels: pad points per butterfly of the first exchange (0 or 1)
     int lds_plane;          // LDS words per plane (re plane, then im plane)
     int conj_in, conj_out;
     int big_shift;          // four-step twiddle split

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <chrono>
 #include <mutex>
+#include <numeric>
 #include <sstream>
 
 #include "planner.h"
@@ -27,8 +28,6 @@ size_t ragged_lds_for(int emax) { return emax == kRaggedHalf ? kRaggedHalfLds : 
 
 constexpr size_t kLdsFloor = 64 * 1024;
 constexpr int64_t kMaxComplexLength = 16384;  // one class's transform fits one workgroup's LDS
-
-int64_t pad16(int64_t x) { return x + (x >> 4); }
 
 
 uint32_t magic_for(int span)
@@ -71,9 +70,21 @@ bool need_lds(const RaggedClassInfo& c)
     return c.sched.radices.size() > 1 || c.variant == kVarR2CEven;
 }
 
+// LDS points per transform of a tile of tpb (RaggedRows, stockham_impl.h), odd so that neighbours start on
+// other banks, and the first exchange's pad: none where the lanes of one transform take banks of their own
+// (64 banks hold 32 points) or where the tile would not fit with it.
+int64_t tile_stride(const RaggedClassInfo& c, int tpb, int* pad)
+{
+    const std::vector<int>& r = c.sched.radices;
+    *pad = (r.size() > 1 && r[0] % 4 == 0 && c.sched.threads * std::gcd(r[0], 32) > 32) ? 1 : 0;
+    if (*pad && (size_t)tpb * (size_t)((c.n + c.n / r[0]) | 1) * 8 > kRaggedLdsLimit) *pad = 0;
+    return (c.n + *pad * (c.n / r[0])) | 1;
+}
+
 size_t class_lds(const RaggedClassInfo& c, int tpb)
 {
-    return need_lds(c) ? (size_t)8 * (size_t)tpb * (size_t)(pad16(c.n) + 1) : 0;
+    int pad = 0;
+    return need_lds(c) ? (size_t)8 * (size_t)tpb * (size_t)tile_stride(c, tpb, &pad) : 0;
 }
 
 // Schedule of a class in the launch of budget kRaggedHalf or kRaggedWide: the fewest-pass radices that
@@ -304,7 +315,7 @@ bool ragged_device_class(const RaggedClassInfo& c, const ClassShape& s, int tpb,
     a.n = (int)c.n;
     a.threads = c.sched.threads;
     a.tpb = tpb;
-    a.lds_tstride = (int)(pad16(c.n) + 1);
+    a.lds_tstride = (int)tile_stride(c, tpb, &a.lds_pad);
     a.lds_plane = tpb * a.lds_tstride;
     a.conj_in = s.conj_in;
     a.conj_out = s.conj_out;
@@ -319,6 +330,8 @@ bool ragged_device_class(const RaggedClassInfo& c, const ClassShape& s, int tpb,
         a.pass[p].span = span;
         a.pass[p].magic = magic_for(span);
         a.pass[p].tw_offset = offs[p];
+        const int64_t nr = c.n / c.sched.radices[p];
+        a.pass[p].read_step = (int)(p == 1 && a.lds_pad ? nr + nr / c.sched.radices[0] : nr);
         span *= c.sched.radices[p];
     }
     rc->variant = c.variant;
@@ -354,7 +367,8 @@ namespace {
 //     30.3 -> 25.8, 4000 to 4096 29.0 -> 27.2 against 32 points per thread, one workgroup per CU;
 //   * else every class on 1024 threads of up to 20 points, one workgroup of 16 wavefronts per CU
 //     (128 VGPRs): 4000 transforms to 16384 101.7 -> 84.2 us, 1000 33.4 -> 29.2, 300 26.4 -> 22.2
-//     against 48 points on 512 threads.  The short classes in a launch of their own at half a CU
+//     against 48 points on 512 threads (79.9, 29.5, 19.4 with the exchange layout of RaggedRows;
+//     4000 to 8192 41.3, 2000 to 2048 on the EMAX-16 budget 13.2 -> 12.7).  The short classes in a launch of their own at half a CU
 //     take 90 us, after the long ones or beside them: the long tiles' last round is nearly empty;
 //   * false where a class fits neither (13, 17, 19 in lengths near 16384): one launch at the largest
 //     register budget, as before.

@@ -74,7 +74,7 @@ __device__ __forceinline__ void ragged_tile(const RaggedArgs& r, const FftArgs& 
                 break;
         }
     }
-    lds_epilogue<kMapRows, EPI>(a, g, lre, lim, tt, tid, 0, live, io);
+    lds_epilogue<kMapRows, EPI, true>(a, g, lre, lim, tt, tid, 0, live, io);
 }
 
 template <int EMAX>

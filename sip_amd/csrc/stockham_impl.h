@@ -217,6 +217,14 @@ template <> struct Dft<12> : DftCT<4, 3> {};
 template <> struct Dft<16> : DftCT<4, 4> {};
 
 // ------------------------------------------------------------------ launch geometry
+// RaggedRows: the ragged kernels (LB) keep a transform's points in LDS in natural order, unpadded except in
+// the first exchange where its radix R0 is a multiple of 4 (writes at a stride of 4 or more points share
+// banks): one pad point per R0 outputs.  R0 divides every later N / R, so both sides of that exchange, and of
+// all others, are a start per butterfly plus a uniform step: one address instruction a point (none in the
+// first pass's writes), where padding every 16 points takes four.  4000 transforms of 64..16384 points issue
+// 13.7 instead of 19.4 million vector instructions with a quarter of the bank conflicts (times: ragged.cpp).
+// The plans' run-time kernels keep the padding every 16: at 96, 384 and 448 points they measured 3 to 12%
+// slower without it, by LDS per workgroup and conflicts between short neighbouring transforms.
 // Sizes a pass needs.  The runtime kernel fills them from kernel arguments; a
 // specialised kernel builds them from template constants, so after inlining every
 // address below folds into immediate offsets (ds_read/ds_write offset fields,
@@ -233,11 +241,12 @@ __device__ __forceinline__ int pad16(int x) { return x + (x >> 4); }
 // LDS slot of element i of transform tt.  Rows: one padded block per transform
 // (one pad word per 16).  Columns: transforms interleaved, row pitch tpb + 1 words, so
 // the slot is linear in i and lanes that take adjacent transforms hit adjacent banks.
-template <int MAP>
+// LIN: the ragged kernels' results, unpadded.
+template <int MAP, bool LIN>
 __device__ __forceinline__ int lds_at(const Geo& g, int tt, int i)
 {
     if constexpr (MAP == kMapRows) {
-        return tt * g.tstride + pad16(i);
+        return tt * g.tstride + (LIN ? i : pad16(i));
     } else {
         return i * (g.tpb + 1) + tt;
     }
@@ -431,7 +440,7 @@ __device__ __forceinline__ float2 lds_point(const float* lre, int at)
 template <int EMAX, int R, int MAP, int PRO, int EPI, bool RT, bool LB = false, bool PRE = false, bool WS = false>
 __device__ __forceinline__ void stockham_pass(const FftArgs& a, Geo g, int span, uint32_t magic, int tw_offset,
                                               bool first, bool last, float* lre, float* lim, int tt, int tid,
-                                              bool live, const Io& io, const float2* twr = nullptr)
+                                              bool live, const Io& io, const float2* twr = nullptr, int read_step = 0)
 {
     float2 v[EMAX];  // pass-local: nothing is carried between passes except through LDS
     constexpr int B = EMAX / R;
@@ -455,6 +464,7 @@ __device__ __forceinline__ void stockham_pass(const FftArgs& a, Geo g, int span,
             return j % span;
         }
     };
+    constexpr bool kLin = RT && LB && MAP == kMapRows;  // see RaggedRows
 
     // 1. gather
     if (first) {
@@ -497,11 +507,17 @@ __device__ __forceinline__ void stockham_pass(const FftArgs& a, Geo g, int span,
         for (int b = 0; b < B; ++b) {
             const int j = tid + b * T;
             if (j < nr) {
-                const int pj = lds_pbase<MAP>(g, j);
+                if constexpr (kLin) {
+                    const float2* at = lc_t + (read_step == nr ? j : j + (int)__umulhi((uint32_t)j, magic));
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int at = lds_rel<MAP, RT>(g, j, pj, r * nr, false);
-                    v[b * R + r] = lc_t[at];
+                    for (int r = 0; r < R; ++r) v[b * R + r] = at[r * read_step];
+                } else {
+                    const int pj = lds_pbase<MAP>(g, j);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int at = lds_rel<MAP, RT>(g, j, pj, r * nr, false);
+                        v[b * R + r] = lc_t[at];
+                    }
                 }
             }
         }
@@ -544,12 +560,24 @@ __device__ __forceinline__ void stockham_pass(const FftArgs& a, Geo g, int span,
             if (j < nr) {
                 const int k = (span > 1) ? kmod(j) : 0;
                 const int base = (j - k) * R + k;
-                const int pb = lds_pbase<MAP>(g, base);
-                const bool base16 = (span == 1) && (R % 16 == 0);  // base = j * R
+                if constexpr (kLin) {
+                    if (span == 1) {  // uniform
+                        float2* at = lc_t + (base + (last ? 0 : a.lds_pad * j));
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int at = lds_rel<MAP, RT>(g, base, pb, r * span, base16);
-                    lc_t[at] = v[b * R + r];
+                        for (int r = 0; r < R; ++r) at[r] = v[b * R + r];
+                    } else {
+                        float2* at = lc_t + base;
+#pragma unroll
+                        for (int r = 0; r < R; ++r) at[r * span] = v[b * R + r];
+                    }
+                } else {
+                    const int pb = lds_pbase<MAP>(g, base);
+                    const bool base16 = (span == 1) && (R % 16 == 0);  // base = j * R
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int at = lds_rel<MAP, RT>(g, base, pb, r * span, base16);
+                        lc_t[at] = v[b * R + r];
+                    }
                 }
             }
         }
@@ -586,8 +614,9 @@ __device__ __forceinline__ void maybe_pass(const FftArgs& a, const Geo& g, int p
         const int span = __builtin_amdgcn_readfirstlane(a.pass[p].span);
         const uint32_t magic = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.pass[p].magic);
         const int tw_offset = __builtin_amdgcn_readfirstlane(a.pass[p].tw_offset);
+        const int read_step = LB ? __builtin_amdgcn_readfirstlane(a.pass[p].read_step) : 0;
         stockham_pass<EMAX, R, MAP, PRO, EPI, true, LB>(a, g, span, magic, tw_offset, p == 0, p == a.passes - 1, lre,
-                                                        lim, tt, tid, live, io);
+                                                        lim, tt, tid, live, io, nullptr, read_step);
     }
     // radices above EMAX are never scheduled: the planner checks radix <= emax before launch
 }
@@ -691,7 +720,7 @@ __device__ __forceinline__ void thread_setup(const FftArgs& a, const Geo& g, int
     }
 }
 
-template <int MAP, int EPI>
+template <int MAP, int EPI, bool LIN = false>
 __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, float* lre, float* lim, int tt, int tid,
                                              int64_t blk, bool live, const Io& io)
 {
@@ -703,8 +732,8 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
             float2* out2 = reinterpret_cast<float2*>(io.out);
             for (int k = tid; 2 * k <= m; k += g.T) {
                 const int km = (k == 0) ? 0 : m - k;
-                const int at0 = lds_at<MAP>(g, tt, k);
-                const int at1 = lds_at<MAP>(g, tt, km);
+                const int at0 = lds_at<MAP, LIN>(g, tt, k);
+                const int at1 = lds_at<MAP, LIN>(g, tt, km);
                 const float2 zk = lds_point(lre, at0);
                 const float2 zm = lds_point(lre, at1);
                 const float2 wk = ldg2(a.tw_aux, k);
@@ -735,7 +764,7 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
             if constexpr (EPI == kEpiTranspose) {
                 float2* ob = reinterpret_cast<float2*>(a.out) + o;
                 for (int i = lane / g.tpb; i < g.n; i += step) {
-                    const int at = lds_at<MAP>(g, tt2, i);
+                    const int at = lds_at<MAP, LIN>(g, tt2, i);
                     ob[i * s] = conj_if(lds_point(lre, at), io.cout);
                 }
             } else {
@@ -743,7 +772,7 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
                 float* obi = a.out_im + o;
                 const float sgn = io.cout ? -1.0f : 1.0f;
                 for (int i = lane / g.tpb; i < g.n; i += step) {
-                    const int at = lds_at<MAP>(g, tt2, i);
+                    const int at = lds_at<MAP, LIN>(g, tt2, i);
                     const float2 x = lds_point(lre, at);
                     obr[i * s] = x.x;
                     obi[i * s] = sgn * x.y;
@@ -763,7 +792,7 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
             float2* out0 = reinterpret_cast<float2*>(a.out) + ob;
             float2* out1 = out0 + a.out_inner;
             for (int i = threadIdx.x; i < g.n; i += g.T * 2) {
-                const int at0 = lds_at<MAP>(g, 0, i), at1 = lds_at<MAP>(g, 1, i);
+                const int at0 = lds_at<MAP, LIN>(g, 0, i), at1 = lds_at<MAP, LIN>(g, 1, i);
                 const float2 u = lds_point(lre, at0);
                 const float2 v = lds_point(lre, at1);
                 out0[i] = conj_if(cadd(u, v), io.cout);
@@ -785,8 +814,8 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
             float2* o2 = o1 + a.out_inner;
             float2* o3 = o2 + a.out_inner;
             for (int i = threadIdx.x; i < g.n; i += g.T * 4) {
-                const int at0 = lds_at<MAP>(g, 0, i), at1 = lds_at<MAP>(g, 1, i);
-                const int at2 = lds_at<MAP>(g, 2, i), at3 = lds_at<MAP>(g, 3, i);
+                const int at0 = lds_at<MAP, LIN>(g, 0, i), at1 = lds_at<MAP, LIN>(g, 1, i);
+                const int at2 = lds_at<MAP, LIN>(g, 2, i), at3 = lds_at<MAP, LIN>(g, 3, i);
                 const float2 u0 = lds_point(lre, at0), u1 = lds_point(lre, at1);
                 const float2 u2 = lds_point(lre, at2), u3 = lds_point(lre, at3);
                 const float2 a0 = cadd(u0, u2), a1 = csub(u0, u2);
@@ -808,7 +837,7 @@ __device__ __forceinline__ void lds_epilogue(const FftArgs& a, const Geo& g, flo
             const int64_t t2 = blk * g.tpb + tt2;
             if (t2 >= a.count) break;  // e only grows: the rest of this thread's elements are past the end
             const int64_t o = (t2 % a.cols) * a.out_inner + (t2 / a.cols) * a.out_outer;
-            const int at = lds_at<MAP>(g, tt2, i);
+            const int at = lds_at<MAP, LIN>(g, tt2, i);
             reinterpret_cast<float2*>(a.out)[o + i] = conj_if(lds_point(lre, at), io.cout);
         }
     }
