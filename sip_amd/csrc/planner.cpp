@@ -1594,15 +1594,49 @@ std::string build_istft_frames(int64_t nfft, int64_t channel, int64_t nframes, B
     return "";
 }
 
+// Where the frames' launch and the overlap-add beat one launch, though it fits.  Measured over 8600
+// batches (nfft 8..1499, 1..64 channels of 2..2000 frames, hop nfft / 16 .. nfft, 2^24 points at most,
+// timed in captured graphs), the one launch is slower than the two in two regions only:
+//   * two groups per workgroup, the first of them transformed for its halo alone (hop about nfft / F).
+//     A batch too small to fill the device then takes the latency of both groups: 1 x 630 x 2 hop 78
+//     12.1 us against 9.5, 37 x 1331 x 3 hop 166 17.7 against 13.8, 4 x 1024 x 50 hop 64 21.9 against
+//     18.8; with more frames the launches' traffic outweighs it (16 x 1024 x 1000 hop 64 ahead again).
+//     Both sides are within 8% of straight lines in the passes, the frame length and the batch.
+//   * groups of 4 frames on more than 8 wavefronts (nfft above 1024 on 129 or more threads per frame:
+//     one workgroup per CU, with 32-byte runs of the spectrum), five or more of them one after
+//     another, while spectrum and frames stay in the device cache (12M points): 12 x 1320 x 325 hop
+//     1015 60 us against 51, 10 x 1386 x 597 hop 1066 93 against 82.
+// Elsewhere 9 of 10 batches are 5 to 60% faster in one launch.
+bool istft_two_launches_faster(const IstftFusedPlan& f, int64_t nfft, int64_t channel, int64_t nframes, int64_t reach)
+{
+    const int F = f.args.fft.tpb, passes = f.args.fft.passes;
+    const double points = 1e-6 * (double)(channel * nframes) * (double)nfft;
+    if (f.args.groups == 2 && reach >= F) {
+        const double tile = (double)(nfft * F) / 1024.0;
+        const double filled = std::min(1.0, (double)f.grid / (double)kNumCUs);
+        const double one = 6.8 + 1.55 * passes + 0.5 * tile * (1.0 + filled);
+        const double two = 5.6 + 1.2 * passes + 2.1 * (double)nfft / 1024.0 + 6.2 * points +
+                           0.36 * (double)std::min(reach, nframes);
+        return one > two;
+    }
+    return F == 4 && F * f.args.fft.threads > 512 && f.args.groups >= 5 && points <= 12.0;
+}
+
 // Where one launch can do: frame lengths whose passes fit 16 points per thread, at most F + 1
 // frames over a sample.  Of the frames per group (16 = 128-byte runs of the spectrum, 8, 4) and
 // the groups per workgroup, the pair of least time: launch rounds x (groups + 1/2) x (what the
-// workgroups of one CU compute per group, about 0.75 us per 1024 points, + 5 us of latency).
-// Separate launches -> one, us: 16 x 1024 x 1000 frames, hop 256 122 -> 84; 16 x 512 x 1000, hop 128
+// workgroups of one CU compute per group, about 0.75 us per 1024 points, + 5 us of latency), or the
+// spectrum at 5 TB/s where that is more: every row of a group is a 128-byte line, also where the
+// group is 4 or 8 frames of it (26 x 440 x 939 hop 146: 83 us in groups of 4, 56 in groups of 16).
+// 128 VGPRs let 16 wavefronts share a CU, but three workgroups of five do not get onto its four
+// SIMDs together: planned as two, 9 x 700 x 1531 hop 175 86 -> 60 us, 12 x 720 x 363 hop 180 28 -> 22.
+// Separate launches -> one, us: 16 x 1024 x 1000 frames, hop 256 122 -> 82; 16 x 512 x 1000, hop 128
 // 67 -> 41; 12 x 720 x 500, hop 180 49 -> 32; 16 x 128 x 1000, hop 32 23 -> 12; 1 x 128 x 50 14.6 -> 11.
 bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, int64_t nframes, int64_t hop,
                        IstftFusedPlan* out)
 {
+    const char* forced = getenv("ASDFFT_ISTFT_FUSED");  // 0: two launches, 1: one wherever it fits (measurement)
+    if (forced != nullptr && forced[0] == '0') return false;
     if (frames.steps.size() != 1 || frames.steps[0].direct || frames.steps[0].shape.emax != 16) return false;
     const FftArgs& step = frames.steps[0].args;
     std::vector<int> radices;
@@ -1621,8 +1655,8 @@ bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, i
         if (T == 0 || T * F > max_block_for(16) || hop > nfft || hop * (F + 1) < nfft) continue;
         const size_t lds = (size_t)(nfft * (F + 1) + nfft - hop + twiddles) * 8 + (size_t)(nfft + hop) * 4;
         if (lds > kLdsLimit) continue;
-        // 128 VGPRs: 16 waves per CU
-        const int64_t per_cu = std::min<int64_t>(16 / ((T * F + 63) / 64), (int64_t)(kLdsLimit / lds));
+        const int64_t waves = (T * F + 63) / 64;
+        const int64_t per_cu = std::min<int64_t>(waves == 5 ? 2 : 16 / waves, (int64_t)(kLdsLimit / lds));
         const int64_t span = nframes + reach - 1;  // hops that hold samples
         for (int64_t groups = 1; groups <= 4096; groups++) {
             const int64_t chunk = groups * F - (reach - 1);
@@ -1631,8 +1665,10 @@ bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, i
             const int64_t grid = channel * chunks;
             const int64_t rounds = (grid + per_cu * kNumCUs - 1) / (per_cu * kNumCUs);
             const int64_t beside = std::min<int64_t>(per_cu, (grid + kNumCUs - 1) / kNumCUs);
-            const double c = (double)rounds * ((double)groups + 0.5) *
-                             (0.75 * (double)(beside * F) * (double)nfft / 1024.0 + 5.0);
+            const double compute = (double)rounds * ((double)groups + 0.5) *
+                                   (0.75 * (double)(beside * F) * (double)nfft / 1024.0 + 5.0);
+            const double lines = (double)(grid * groups) * (double)nfft * 128.0 / 5e6;
+            const double c = std::max(compute, lines);
             if (c < cost && grid <= 0x7fffffff) {
                 cost = c;
                 best.args.groups = (int)groups;
@@ -1648,6 +1684,7 @@ bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, i
         }
     }
     if (best.grid == 0) return false;
+    if (forced == nullptr && istft_two_launches_faster(best, nfft, channel, nframes, reach)) return false;
     best.args.halo = (int)(reach - 1);
     best.args.hop_magic = (uint32_t)(((uint64_t)1 << 32) / (uint64_t)hop + 1);
     std::ostringstream os;
