@@ -104,7 +104,7 @@ __global__ void __launch_bounds__((bl_block<M / kBlPoints>())) bluestein_kernel(
     const int tt = threadIdx.x / T;
     const int tid = threadIdx.x % T;
     float2* lds = reinterpret_cast<float2*>(smem) + tt * (M + M / 16 + 1);
-    const int64_t t = (int64_t)blockIdx.x * a.tpb + tt;
+    const int64_t t = dft_block(a) * a.tpb + tt;
     const bool live = t < a.count;
     const int n = live ? a.n : 0;  // lanes of a transform past the batch load and store nothing
     int64_t ib = t * a.in_dist;
@@ -168,7 +168,7 @@ std::vector<int> bluestein_radices(int64_t m, bool second)
     return {};
 }
 
-hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, hipStream_t stream)
+hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, dim3 grid, hipStream_t stream)
 {
 #define ASDFFT_BL_LAUNCH(M, R1, RL, F, I)                                                                       \
     if (args.m == M) {                                                                                          \
@@ -179,7 +179,7 @@ hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, hipStream
             hipError_t e = raise_lds_limit_once(reinterpret_cast<const void*>(kern), raised);                   \
             if (e != hipSuccess) return e;                                                                      \
         }                                                                                                       \
-        hipLaunchKernelGGL(kern, dim3((unsigned)s.grid), dim3((unsigned)s.block), s.lds_bytes, stream, args);   \
+        hipLaunchKernelGGL(kern, grid, dim3((unsigned)s.block), s.lds_bytes, stream, args);                     \
         return hipGetLastError();                                                                               \
     }
     ASDFFT_BLUESTEIN(ASDFFT_BL_LAUNCH)

@@ -9,6 +9,12 @@
 
 namespace asdfft {
 
+// Index of the workgroup: the grid has rows of row_blocks (launch_dft_direct).
+__device__ __forceinline__ int64_t dft_block(const DftArgs& a)
+{
+    return (int64_t)blockIdx.y * a.row_blocks + blockIdx.x;
+}
+
 __device__ __forceinline__ float2 dft_load(const DftArgs& a, int64_t base, int i)
 {
     const float2* in2 = reinterpret_cast<const float2*>(a.in);

@@ -11,7 +11,7 @@ namespace asdfft {
 // Length 1: every element through its layout's load and store (an identity axis, a plan of N == 1).
 __global__ void __launch_bounds__(256) dft_unit_kernel(const DftArgs a)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = dft_block(a) * 256 + threadIdx.x;
     if (t >= a.count) return;
     dft_store(a, t * a.out_dist, 0, dft_load(a, (t % a.in_cols) + (t / a.in_cols) * a.in_dist, 0));
 }
@@ -33,7 +33,7 @@ __global__ void __launch_bounds__(256) dft_pairs_kernel(const DftArgs a)
     __shared__ float2 roots[N];
     const int tt = threadIdx.x / kPairLanes;
     const int k = threadIdx.x % kPairLanes;
-    const int64_t t = (int64_t)blockIdx.x * (256 / kPairLanes) + tt;
+    const int64_t t = dft_block(a) * (256 / kPairLanes) + tt;
     const bool live = t < a.count && k <= H;
     if (threadIdx.x < N) roots[threadIdx.x] = reinterpret_cast<const float2*>(a.roots)[threadIdx.x];
     if (live) {
@@ -66,14 +66,21 @@ bool dft_pairs_length(int64_t n) { return n == 23 || n == 29 || n == 31; }
 
 int dft_pairs_per_block() { return 256 / kPairLanes; }
 
-hipError_t launch_dft_direct(const LaunchShape& s, const DftArgs& args, hipStream_t stream)
+hipError_t launch_dft_direct(const LaunchShape& s, const DftArgs& dft, hipStream_t stream)
 {
-    if (s.grid <= 0 || s.grid > 0x7fffffff || s.block <= 0 || s.block > 1024) return hipErrorInvalidConfiguration;
-    if (args.n > 1 && !dft_pairs_length(args.n)) return launch_bluestein(s, args, stream);
+    // A workgroup holds few of these transforms (16 of 23 points), and one dimension of a grid less
+    // than 2^32 threads: 2^28 transforms of 23 points, 49 GB.  Rows of up to 65536 workgroups, of
+    // equal length, so that at most one workgroup a row has nothing to do.
+    const int64_t rows = (s.grid + 65535) / 65536;
+    if (s.grid <= 0 || rows > 65535 || s.block <= 0 || s.block > 1024) return hipErrorInvalidConfiguration;
+    DftArgs args = dft;
+    args.row_blocks = (int)((s.grid + rows - 1) / rows);
+    const dim3 grid((unsigned)args.row_blocks, (unsigned)rows);
+    if (args.n > 1 && !dft_pairs_length(args.n)) return launch_bluestein(s, args, grid, stream);
     if (s.block != 256) return hipErrorInvalidConfiguration;
     auto kern = args.n == 23 ? dft_pairs_kernel<23> : args.n == 29 ? dft_pairs_kernel<29>
               : args.n == 31 ? dft_pairs_kernel<31> : dft_unit_kernel;
-    hipLaunchKernelGGL(kern, dim3((unsigned)s.grid), dim3((unsigned)s.block), 0, stream, args);
+    hipLaunchKernelGGL(kern, grid, dim3((unsigned)s.block), 0, stream, args);
     return hipGetLastError();
 }
 

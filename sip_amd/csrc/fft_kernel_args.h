@@ -137,6 +137,7 @@ struct DftArgs {
     int n;
     int m;                  // convolution length M
     int tpb;
+    int row_blocks;         // workgroups of one grid row (set at the launch)
     int conj_in, conj_out;
     int prologue, epilogue; // kProComplex/kProReal/kProHerm/kProPlanar, kEpiComplex/kEpiHalf/kEpiReal/kEpiPlanar
     int64_t count;
