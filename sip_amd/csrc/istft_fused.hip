@@ -270,7 +270,7 @@ bool istft_fused_radix(int radix)
 hipError_t launch_istft_fused(const IstftFusedArgs& args, int64_t grid, size_t lds_bytes, hipStream_t stream)
 {
     const int block = args.fft.tpb * args.fft.threads;
-    if (grid <= 0 || grid > 0x7fffffff || block <= 0 || block > 1024 || args.ola.hop <= 0 || args.ola.hop > args.fft.n ||
+    if (grid <= 0 || block <= 0 || block > 1024 || grid > 0xffffffff / block || args.ola.hop <= 0 || args.ola.hop > args.fft.n ||
         args.groups <= 0 || args.chunk_frames <= 0)
         return hipErrorInvalidValue;
     LaunchShape s;

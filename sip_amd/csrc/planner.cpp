@@ -1669,7 +1669,7 @@ bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, i
                                    (0.75 * (double)(beside * F) * (double)nfft / 1024.0 + 5.0);
             const double lines = (double)(grid * groups) * (double)nfft * 128.0 / 5e6;
             const double c = std::max(compute, lines);
-            if (c < cost && grid <= 0x7fffffff) {
+            if (c < cost && grid * T * F <= 0xffffffff) {  // threads of a launch
                 cost = c;
                 best.args.groups = (int)groups;
                 best.args.chunk_frames = chunk;

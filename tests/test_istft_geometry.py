@@ -36,6 +36,21 @@ def test_route(shape, frames):
         assert f"istft fused frames/group={frames} " in text, text
 
 
+@pytest.mark.parametrize("shape", [(1 << 21, 1024, 2, 64), (1 << 22, 1024, 2, 64), (1 << 23, 1024, 2, 256)], ids=str)
+def test_launch_stays_within_2_to_32_threads(shape):
+    """Where the one launch would pass them (one workgroup of 1024 threads for two frames of a
+    channel, 2^22 channels: 69 GB), the two launches stay."""
+    import re
+
+    from sip_amd import Istft
+    p = Istft(*shape)
+    text = p.describe()
+    p.close()
+    m = re.search(r"istft fused frames/group=(\d+) T=(\d+) .*grid=(\d+)", text)
+    assert (m is None) == (shape == (1 << 22, 1024, 2, 64)), text
+    assert m is None or math.prod(map(int, m.groups())) < 1 << 32, text
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", [(1, 630, 2, 78), (3, 1024, 5, 64), (2, 1320, 33, 1015), (9, 700, 41, 175), (5, 440, 37, 146)],
                          ids=str)
