@@ -382,8 +382,9 @@ bool single_launch_geometry(const RaggedOptions& opt, std::vector<RaggedClassInf
         fits16 = fits16 && ragged_schedule(&own, f != opt.fixed.end() ? &f->second : nullptr, &unsupported).empty() &&
                  own.emax <= 16;
     }
-    if (fits16) return false;
+    if (fits16 && opt.budget == 0) return false;
     for (int emax : {kRaggedHalf, kRaggedWide}) {
+        if (opt.budget != 0 && opt.budget != emax) continue;
         std::vector<RaggedClassInfo> sized = *classes;
         bool fits = true;
         for (RaggedClassInfo& c : sized) {
@@ -464,6 +465,10 @@ std::string build_once(const std::vector<RaggedEntry>& entries, const RaggedOpti
 
     // ---- per-class schedules
     const bool sized = opt.one_launch && !opt.wide16 && opt.sized && single_launch_geometry(opt, &plan->classes);
+    plan->sized_budget = 0;
+    if (sized) {
+        for (const RaggedClassInfo& c : plan->classes) plan->sized_budget = std::max(plan->sized_budget, c.emax);
+    }
     for (size_t ci = 0; ci < plan->classes.size() && !sized; ci++) {
         RaggedClassInfo& c = plan->classes[ci];
         auto f = opt.fixed.find(c.key);
@@ -842,7 +847,11 @@ double time_exec(RaggedPlan& p, void* in, void* out, hipStream_t s, int reps)
 
 std::string cache_key(int device, const std::string& key, const RaggedOptions& opt)
 {
-    return std::to_string(device) + "|" + key + "|" + std::to_string(opt.block16) + "|" + std::to_string(opt.block32);
+    // and the form that decides which kernel times it
+    std::ostringstream os;
+    os << device << "|" << key << "|" << opt.block16 << "|" << opt.block32 << "|" << opt.one_launch << opt.wide16
+       << opt.sized << "|" << opt.budget;
+    return os.str();
 }
 
 // Times every candidate schedule of class c (alone, replicated to about kTuneBytes) and
@@ -870,7 +879,7 @@ ClassSchedule tune_class(const RaggedClassInfo& c, const RaggedOptions& base, Sc
         o.fixed[c.key] = cand;
         RaggedPlan p;
         bool unsup = false;
-        if (!build_once({e}, o, &p, &unsup).empty() || !p.ready) continue;
+        if (!build_once({e}, o, &p, &unsup).empty() || !p.ready || p.sized_budget != o.budget) continue;
         const double ms = time_exec(p, scratch.in, scratch.out, s, kTuneReps);
         (*timed)++;
         if (ms < best_ms) {
@@ -939,6 +948,10 @@ std::string build_ragged(const std::vector<RaggedEntry>& entries, const RaggedOp
     hipStream_t s = nullptr;
     if (hipStreamCreate(&s) != hipSuccess) return build_once(entries, plain, plan, unsupported);
     int timed = 0;
+    // Classes are timed, and the tuned plan runs, in the batch's own kernel where it is a sized launch;
+    // elsewhere each in the kernel of its own register budget.
+    plain.sized = probe.sized_budget != 0;
+    plain.budget = probe.sized_budget;
     RaggedOptions tuned = plain;
     {
         Scratch scratch;
@@ -950,8 +963,9 @@ std::string build_ragged(const std::vector<RaggedEntry>& entries, const RaggedOp
             if (it == tune_cache().end()) it = tune_cache().emplace(ck, tune_class(c, plain, scratch, s, &timed)).first;
             tuned.fixed[c.key] = it->second;
         }
-        // workgroup size of each launch, timed on the whole batch with the tuned schedules
-        if (opt.block16 == 0 || opt.block32 == 0) {
+        // workgroup size of each launch, timed on the whole batch with the tuned schedules (a sized
+        // launch's is fixed by its budget)
+        if (!plain.sized && (opt.block16 == 0 || opt.block32 == 0)) {
             size_t need = std::max(probe.in_extent, probe.out_extent);
             if (scratch.ensure(need)) {
                 double best = 1e30;
@@ -985,8 +999,9 @@ std::string build_ragged(const std::vector<RaggedEntry>& entries, const RaggedOp
     plan->tune_timed = timed;
     plan->tune_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     std::ostringstream os;
-    os << plan->describe << "  autotuned: " << timed << " timings in " << (int)plan->tune_ms << " ms, block16="
-       << tuned.block16 << "\n";
+    os << plan->describe << "  autotuned: " << timed << " timings in " << (int)plan->tune_ms << " ms";
+    if (!plain.sized) os << ", block16=" << tuned.block16;
+    os << "\n";
     plan->describe = os.str();
     return why;
 }

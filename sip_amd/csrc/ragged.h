@@ -64,6 +64,8 @@ struct RaggedOptions {
     bool one_launch = true;  // every class in one launch at the largest register budget (false:
                              // one concurrent launch per register budget)
     bool sized = true;       // one launch: its geometry by the longest class (single_launch_geometry)
+    int budget = 0;          // a sized launch's budget (0: the smallest that holds every class); a class
+                             // is tuned alone in the kernel that its batch runs
     bool wide16 = false;     // EMAX-16 schedules of up to 1024 threads per transform before larger budgets
                              // (the EMAX-16 classes then take a launch of their own: two launches)
     int block16 = 0;        // workgroup size of the EMAX-16 launch (0: automatic)
@@ -104,6 +106,7 @@ struct RaggedPlan {
     std::vector<RaggedEntry> entries;
     double tune_ms = 0;            // plan-time autotuning wall time (0 when not tuned)
     int tune_timed = 0;            // candidate schedules timed
+    int sized_budget = 0;          // budget of a sized single launch (0: not sized)
     std::vector<RaggedClassInfo> classes;
     std::vector<RaggedLaunchPlan> launches;
     std::vector<int64_t> offsets;  // host copy of the offset table
