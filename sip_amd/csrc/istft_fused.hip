@@ -273,10 +273,6 @@ hipError_t launch_istft_fused(const IstftFusedArgs& args, int64_t grid, size_t l
     if (grid <= 0 || block <= 0 || block > 1024 || grid > 0xffffffff / block || args.ola.hop <= 0 || args.ola.hop > args.fft.n ||
         args.groups <= 0 || args.chunk_frames <= 0)
         return hipErrorInvalidValue;
-    LaunchShape s;
-    s.grid = grid;
-    s.block = block;
-    s.lds_bytes = lds_bytes;
     if (lds_bytes > 65536) {
         static std::atomic<uint64_t> raised{0};
         const hipError_t e = raise_lds_limit_once(reinterpret_cast<const void*>(istft_fused_kernel), raised);

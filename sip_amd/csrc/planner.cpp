@@ -111,26 +111,9 @@ struct Config {
 // Rows mapping: lanes along a transform; several short transforms per workgroup.
 // want_tpb > 0 asks for that many transforms per workgroup (transposed stores need
 // >= 16 adjacent transforms for 128-byte runs) and may use the whole LDS.
-// The fewest-pass radix sequence, or, when its largest per-thread share does not fit
-// the register budgets, the first radix multiset (more passes) that does.
-std::vector<int> fitting_radices(int64_t n)
-{
-    std::vector<int> r = choose_radices(n);
-    if (r.empty()) return r;
-    for (int emax : {16, 32}) {
-        if (threads_for(n, r, emax) > 0) return r;
-    }
-    for (const std::vector<int>& alt : radix_multisets(n, 3, 64)) {
-        for (int emax : {16, 32}) {
-            if (threads_for(n, alt, emax) > 0) return alt;
-        }
-    }
-    return r;
-}
-
 bool rows_config(int64_t n, int64_t count, bool epi_lds, int want_tpb, int variant, Config* c)
 {
-    std::vector<int> radices = fitting_radices(n);
+    std::vector<int> radices = choose_radices(n);
     if (radices.empty()) return false;
     // 4096-point C2C rows with at most one transform per CU: four radix-8 passes on 512 threads
     // x 8 points instead of three radix-16 passes on 256 x 16, so each CU has twice the waves to
@@ -242,7 +225,7 @@ int split_variant_of(int variant)
 // Column mapping: lanes across adjacent transforms (columns) for coalesced strided access.
 bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_split = false)
 {
-    std::vector<int> radices = fitting_radices(n);
+    std::vector<int> radices = choose_radices(n);
     if (radices.empty()) return false;
     // ASDFFT_COLS="n:emax:T:tpb" forces a column geometry that has a specialised kernel
     // (measurement of alternatives)

@@ -44,10 +44,6 @@ std::vector<int> choose_radices(int64_t n);
 // every radix is <= 16, then by butterfly cost.  At most `limit` of them.
 std::vector<std::vector<int>> radix_multisets(int64_t n, int extra, int limit);
 
-// choose_radices(n), or when that sequence needs more threads per transform than a
-// workgroup holds, the fewest-pass alternative multiset that fits.
-std::vector<int> fitting_radices(int64_t n);
-
 // Threads per transform needed to cover every pass with EMAX/R butterflies per
 // thread, or 0 when this EMAX cannot hold a radix of the sequence or the
 // transform does not fit the EMAX's workgroup limit.
