@@ -108,6 +108,37 @@ struct Config {
     bool split = false;  // one-plane LDS exchange (the variant's specialised split kernel)
 };
 
+// Workgroups of one transform on `threads` threads and `lds` bytes that a CU holds at once.  A SIMD
+// holds 4 wavefronts of the EMAX-32 kernels (95 to 121 VGPRs); of the EMAX-16 ones 8 (61 to 63), 6 of
+// the even real kernels (77, 78), 5 of the planar rows (82), 7 of planar rows into complex (65).
+int64_t resident_rows(int variant, int emax, int threads, size_t lds)
+{
+    int waves = 4;
+    if (emax <= 16) {
+        waves = variant == kVarR2CEven || variant == kVarC2REven ? 6
+              : variant == kVarRowsSep ? 5 : variant == kVarRowsSepIn ? 7 : 8;
+    }
+    const int64_t by_waves = waves / ((threads + 255) / 256);
+    return std::max<int64_t>(1, std::min<int64_t>(by_waves, (int64_t)(kLdsLimit / std::max<size_t>(lds, 1))));
+}
+
+// Launches of more transforms than CUs whose EMAX-16 workgroup (threads, lds) fills a CU alone while
+// several EMAX-32 ones share it: true where those are quicker.  Three of them are (planar rows of 4900
+// to 6500 points: 5670 x 694 30.7 us -> 25.0, 5040 x 2902 26%, 8 of 10 batches); two where they need one
+// round and EMAX 16 two (planar rows 8320 x 272 and C2R 13860 x 285 15%, 7700..9400 x 260..500 4 to
+// 15%), and for R2C of more than three rounds (18000 x 2872 12%, 18144 x 952 9%).  Elsewhere the two are
+// level within 10% either way, EMAX 16 ahead at three rounds.
+bool rows_share_a_cu(int64_t n, int64_t count, int variant, const std::vector<int>& radices, int threads, size_t lds)
+{
+    if (threads <= 256 || count <= kNumCUs || !has_instance(variant, 32) || resident_rows(variant, 16, threads, lds) > 1 ||
+        find_static(variant, 16, (int)n, threads, 0, radices.data(), (int)radices.size()) >= 0)
+        return false;
+    const int threads32 = threads_for(n, radices, 32);
+    if (threads32 == 0 || threads32 > 512) return false;
+    const int64_t beside = resident_rows(variant, 32, threads32, lds);
+    return beside >= 3 || (beside == 2 && (count <= 2 * kNumCUs || (variant == kVarR2CEven && count > 3 * kNumCUs)));
+}
+
 // Rows mapping: lanes along a transform; several short transforms per workgroup.
 // want_tpb > 0 asks for that many transforms per workgroup (transposed stores need
 // >= 16 adjacent transforms for 128-byte runs) and may use the whole LDS.
@@ -185,7 +216,9 @@ bool rows_config(int64_t n, int64_t count, bool epi_lds, int want_tpb, int varia
         // most 512 threads against EMAX 16: C2C 3402 32.2 -> 19.5 us, 4320 24.0 -> 20.0, 7000 33.8
         // -> 25.4, 10240 33.1 -> 26.7; R2C 6804 21.6 -> 16.3, C2R 12150 24.9 -> 20.3; a tenth of
         // that many points 13 -> 9 us; 8192 and 16384 (specialised either way) 2-10% faster.
-        if (want_tpb <= 0) break;
+        if (want_tpb > 0) continue;
+        if (emax > 16 || !rows_share_a_cu(n, count, variant, radices, T, lds)) break;
+        found = false;
     }
     if (found && wide8 && best.emax == 16) {
         best.threads = wide->threads;
