@@ -295,10 +295,14 @@ bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_s
     // at EMAX 16, 882 62.5 -> 31, 1500 51.6 (8) -> 38.4 (4), 324 39.3 (EMAX 32) -> 28.9.  32-byte
     // runs of 4 columns, with neighbours on one XCD, still beat one workgroup per CU at 8; from
     // HBM (2^24 points) the two are level.  A specialised instance of the same width goes first.
+    // A four-step transform's first pass keeps EMAX-32 workgroups within 512 threads: with 1024 a single
+    // long transform is split into lengths of up to 2240 points whose 16 columns leave it 43 to 72
+    // workgroups (r2c 1462050 48.0 against 36.6 us, c2c 795600 37.2 / 31.9, 1290240 45.9 / 41.2).
+    const bool twiddle = variant == kVarColsTwiddle || variant == kVarColsTwiddleSep;
     const auto cols_fit = [&](int tpb, int emax, size_t cap) {
         if (!has_instance(variant, emax)) return false;
         const int T = threads_for(n, radices, emax);
-        if (T == 0 || tpb * T > max_block_for(emax)) return false;
+        if (T == 0 || tpb * T > (twiddle && emax > 16 ? 512 : max_block_for(emax))) return false;
         const int64_t plane = n * (tpb + 1);  // column layout: row pitch tpb + 1 words
         const bool need_lds = radices.size() > 1 || variant == kVarColsToRows;  // (epilogue via LDS)
         const size_t lds = need_lds ? (size_t)(8 * plane) : 0;

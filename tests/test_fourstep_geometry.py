@@ -1,0 +1,42 @@
+"""First passes of four-step transforms (cols_config in planner.cpp): workgroups of 32 points a thread stay
+within 512 threads, and the lengths that this moves against the FP64 oracle at relative L2 <= 1e-6 *
+log2(N) per transform."""
+import math
+import re
+
+import numpy as np
+import pytest
+
+LENGTHS = [468160, 536085, 795600, 841568, 1290240, 1462050]
+
+
+def first_pass(n, batch):
+    from sip_amd.fft import Plan
+    p = Plan("c2c", (n,), batch)
+    text = p.describe()
+    p.close()
+    return [int(v) for v in re.search(r"variant=6 n=(\d+) .*?emax=(\d+) T=(\d+) tpb=(\d+) block=(\d+)", text).groups()], text
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+@pytest.mark.parametrize("batch", [1, 9])
+def test_first_pass_stays_within_its_threads(n, batch):
+    (_, emax, threads, tpb, block), text = first_pass(n, batch)
+    assert block == threads * tpb <= (1024 if emax == 16 else 512), text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", LENGTHS)
+def test_long_lengths_match_oracle(oracle, n):
+    import torch
+
+    from oracle.oracle import rel_l2_per_row
+    from sip_amd.fft import Plan
+    rng = np.random.default_rng(n)
+    x = (rng.uniform(-1, 1, (2, n)) + 1j * rng.uniform(-1, 1, (2, n))).astype(np.complex64)
+    p = Plan("c2c", (n,), 2)
+    try:
+        got = p.execute(torch.from_numpy(x).cuda()).cpu().numpy()
+    finally:
+        p.close()
+    assert rel_l2_per_row(got, oracle.c2c(x, False)).max() <= 1e-6 * math.log2(n)
