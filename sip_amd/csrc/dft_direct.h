@@ -46,14 +46,16 @@ __device__ __forceinline__ void dft_store(const DftArgs& a, int64_t base, int k,
         reinterpret_cast<float*>(a.out)[base + k] = x.x;
         return;
     }
-    // A real input's bins 0 and n/2 are real.  The chirp transform leaves rounding there; the product
-    // keeps what is not finite visible in both parts.
-    if (a.epilogue == kEpiHalf && (k == 0 || 2 * k == a.n)) x.y = 0.0f * x.x + 0.0f;
     if (a.conj_out) x.y = -x.y;
     if (a.epilogue == kEpiPlanar) {
         reinterpret_cast<float*>(a.out)[base + k] = x.x;
         a.out_im[base + k] = x.y;
-    } else if (a.epilogue != kEpiHalf || 2 * k <= a.n) {
+    } else if (a.epilogue != kEpiHalf) {
+        reinterpret_cast<float2*>(a.out)[base + k] = x;
+    } else if (2 * k <= a.n) {
+        // A real input's bins 0 and n/2 are real.  The chirp transform leaves rounding there; the product
+        // keeps what is not finite visible in both parts.
+        if (k == 0 || 2 * k == a.n) x.y = 0.0f * x.x + 0.0f;
         reinterpret_cast<float2*>(a.out)[base + k] = x;
     }
 }
