@@ -1,4 +1,5 @@
-// Transforms of lengths 1, 23, 29 and 31, and the launch dispatcher for the Stockham variants.
+// Transforms of lengths 1, 23, 29, 31 and of others to 127 as sums over pairs, and the launch dispatcher
+// for the Stockham variants.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -62,6 +63,61 @@ __global__ void __launch_bounds__(256) dft_pairs_kernel(const DftArgs a)
     if (k > 0) dft_store(a, t * a.out_dist, N - k, make_float2(p.x + s.y, p.y - s.x));
 }
 
+// The same sum at any length to 127, one transform per wavefront (lane k: X_k and X_(n-k)).  Its 63 terms
+// at most take less than the passes of a chirp transform until the batch fills the chip: 43 x 4 4.3 us
+// (chirp 6.2, the sum over all terms before that 4.4), 127 x 4 5.5 (7.0), 127 x 2048 7.0 (8.0).  Bound by
+// the latency of the loads and of one LDS read of a root and a pair per term.
+__global__ void __launch_bounds__(64) dft_sum_kernel(const DftArgs a)
+{
+    __shared__ float4 pairs[64];
+    __shared__ float2 roots[kMaxSum];
+    const int64_t t = dft_block(a);
+    if (t >= a.count) return;  // the whole workgroup
+    const int n = a.n, half = n / 2, k = threadIdx.x;
+    const bool twice = k > 0 && 2 * k < n;  // x_k and x_(n-k) are two elements
+    for (int m = threadIdx.x; m < n; m += 64) roots[m] = reinterpret_cast<const float2*>(a.roots)[m];
+    if (k <= half) {
+        const int64_t ib = (t % a.in_cols) + (t / a.in_cols) * a.in_dist;
+        const float2 x = dft_load(a, ib, k);
+        float4 v = make_float4(x.x, x.y, 0.0f, 0.0f);
+        if (twice) {
+            const float2 y = dft_load(a, ib, n - k);
+            v = make_float4(x.x + y.x, x.y + y.y, x.x - y.x, x.y - y.y);
+        }
+        pairs[k] = v;
+    }
+    __syncthreads();
+    if (k > half) return;
+    // four running sums, added at the end: their error is half that of one
+    float2 p[4], s[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = s[q] = make_float2(0.0f, 0.0f);
+    int m = 0;
+    const auto add = [&](int i, int q) __attribute__((always_inline)) {
+        m += k;
+        if (m >= n) m -= n;
+        const float2 w = roots[m];  // cos, -sin
+        const float4 v = pairs[i];
+        p[q].x += v.x * w.x;
+        p[q].y += v.y * w.x;
+        s[q].x += v.z * w.y;
+        s[q].y += v.w * w.y;
+    };
+    int i = 1;
+    for (; i + 3 <= half; i += 4) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) add(i + q, q);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        if (i + q <= half) add(i + q, q);
+    }
+    const float2 u = cadd(make_float2(pairs[0].x, pairs[0].y), cadd(cadd(p[0], p[1]), cadd(p[2], p[3])));
+    const float2 d = cadd(cadd(s[0], s[1]), cadd(s[2], s[3]));
+    dft_store(a, t * a.out_dist, k, make_float2(u.x - d.y, u.y + d.x));
+    if (twice) dft_store(a, t * a.out_dist, n - k, make_float2(u.x + d.y, u.y - d.x));
+}
+
 bool dft_pairs_length(int64_t n) { return n == 23 || n == 29 || n == 31; }
 
 int dft_pairs_per_block() { return 256 / kPairLanes; }
@@ -76,9 +132,10 @@ hipError_t launch_dft_direct(const LaunchShape& s, const DftArgs& dft, hipStream
     DftArgs args = dft;
     args.row_blocks = (int)((s.grid + rows - 1) / rows);
     const dim3 grid((unsigned)args.row_blocks, (unsigned)rows);
-    if (args.n > 1 && !dft_pairs_length(args.n)) return launch_bluestein(s, args, grid, stream);
-    if (s.block != 256) return hipErrorInvalidConfiguration;
-    auto kern = args.n == 23 ? dft_pairs_kernel<23> : args.n == 29 ? dft_pairs_kernel<29>
+    const bool sum = args.m == 0 && args.n > 1 && !dft_pairs_length(args.n);
+    if (args.m > 0) return launch_bluestein(s, args, grid, stream);
+    if (s.block != (sum ? 64 : 256) || (sum && args.n > kMaxSum)) return hipErrorInvalidConfiguration;
+    auto kern = sum ? dft_sum_kernel : args.n == 23 ? dft_pairs_kernel<23> : args.n == 29 ? dft_pairs_kernel<29>
               : args.n == 31 ? dft_pairs_kernel<31> : dft_unit_kernel;
     hipLaunchKernelGGL(kern, grid, dim3((unsigned)s.block), 0, stream, args);
     return hipGetLastError();

@@ -88,6 +88,7 @@ int find_static(int variant, int emax, int n, int threads, int tpb, const int* r
 hipError_t launch_dft_direct(const LaunchShape& s, const DftArgs& args, hipStream_t stream);
 bool dft_pairs_length(int64_t n);  // 23, 29, 31: the sum over pairs (dft_pairs_kernel)
 int dft_pairs_per_block();
+constexpr int kMaxSum = 127;  // longest length of dft_sum_kernel
 hipError_t launch_bluestein(const LaunchShape& s, const DftArgs& args, dim3 grid, hipStream_t stream);
 // Radices of the first / second transform of convolution length m (empty: no kernel).
 std::vector<int> bluestein_radices(int64_t m, bool second);
