@@ -298,11 +298,13 @@ bool cols_config(int64_t n, int64_t count, int variant, Config* c, bool prefer_s
     // A four-step transform's first pass keeps EMAX-32 workgroups within 512 threads: with 1024 a single
     // long transform is split into lengths of up to 2240 points whose 16 columns leave it 43 to 72
     // workgroups (r2c 1462050 48.0 against 36.6 us, c2c 795600 37.2 / 31.9, 1290240 45.9 / 41.2).
-    const bool twiddle = variant == kVarColsTwiddle || variant == kVarColsTwiddleSep;
+    // So do shifted columns (lengths of factors 17 and 19): 1156 x 300 x 15 63.1 against 52.0 us, 1197 x 85
+    // 21.1 / 17.8.  Plain columns of the same lengths are level or quicker with more threads.
+    const bool narrow = variant == kVarColsTwiddle || variant == kVarColsTwiddleSep || variant == kVarColsShiftOut;
     const auto cols_fit = [&](int tpb, int emax, size_t cap) {
         if (!has_instance(variant, emax)) return false;
         const int T = threads_for(n, radices, emax);
-        if (T == 0 || tpb * T > (twiddle && emax > 16 ? 512 : max_block_for(emax))) return false;
+        if (T == 0 || tpb * T > (narrow && emax > 16 ? 512 : max_block_for(emax))) return false;
         const int64_t plane = n * (tpb + 1);  // column layout: row pitch tpb + 1 words
         const bool need_lds = radices.size() > 1 || variant == kVarColsToRows;  // (epilogue via LDS)
         const size_t lds = need_lds ? (size_t)(8 * plane) : 0;

@@ -1,6 +1,6 @@
-"""First passes of four-step transforms (cols_config in planner.cpp): workgroups of 32 points a thread stay
-within 512 threads, and the lengths that this moves against the FP64 oracle at relative L2 <= 1e-6 *
-log2(N) per transform."""
+"""First passes of four-step transforms and shifted columns (cols_config in planner.cpp): workgroups of 32
+points a thread stay within 512 threads, and what this moves against the FP64 oracle at relative L2 <=
+1e-6 * log2(N) per transform."""
 import math
 import re
 
@@ -40,3 +40,33 @@ def test_long_lengths_match_oracle(oracle, n):
     finally:
         p.close()
     assert rel_l2_per_row(got, oracle.c2c(x, False)).max() <= 1e-6 * math.log2(n)
+
+
+SHIFTED = [(1156, 30), (1197, 85), (833, 75)]
+
+
+@pytest.mark.parametrize("dims", SHIFTED)
+def test_shifted_columns_stay_within_their_threads(dims):
+    from sip_amd.fft import Plan
+    p = Plan("c2c", dims, 2, in_shift="ifft", out_shift="fft")
+    text = p.describe()
+    p.close()
+    assert int(re.search(r"variant=18 .*?block=(\d+)", text).group(1)) <= 512, text
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", SHIFTED)
+def test_shifted_columns_match_oracle(oracle, dims):
+    import torch
+
+    from oracle.oracle import rel_l2_per_row
+    from sip_amd.fft import Plan
+    rng = np.random.default_rng(dims[0])
+    x = (rng.uniform(-1, 1, (2,) + dims) + 1j * rng.uniform(-1, 1, (2,) + dims)).astype(np.complex64)
+    p = Plan("c2c", dims, 2, in_shift="ifft", out_shift="fft")
+    try:
+        got = p.execute(torch.from_numpy(x).cuda()).cpu().numpy()
+    finally:
+        p.close()
+    want = np.fft.fftshift(oracle.c2c_nd(np.fft.ifftshift(x, (1, 2)), 2, False), (1, 2))
+    assert rel_l2_per_row(got, want, 2).max() <= 1e-6 * math.log2(dims[0] * dims[1])
