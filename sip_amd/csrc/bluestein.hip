@@ -1,4 +1,5 @@
-// Lengths with prime factors above 19 (32 < n <= 8192): the chirp transform (L. Bluestein, 1970).
+// Lengths with prime factors above 19 (32 < n <= 8192, of those to 127 the batches above 2048): the chirp
+// transform (L. Bluestein, 1970).
 //
 //   X_k = w_k sum_i (x_i w_i) conj(w_(k - i)),   w_k = e^(-i pi k^2 / n)
 //

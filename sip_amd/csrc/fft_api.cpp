@@ -1179,9 +1179,10 @@ extern "C" int32_t asdFftExtMakePlanRagged(void* handle, const asdFftExtRaggedEn
     opt.graph = (flags & ASDFFT_RAGGED_GRAPH) != 0;
     opt.autotune = (flags & ASDFFT_RAGGED_AUTOTUNE) != 0;
     opt.one_launch = (flags & ASDFFT_RAGGED_PER_BUDGET) == 0;
-    // ASDFFT_RAGGED_WIDE16=1: the EMAX-16 classes on wide workgroups (up to 1024 threads per
-    // transform) in a launch of their own beside the single launch of the others (measured
-    // within 3% of the single launch: 100.6 vs 103.3 us on the 4000-transform workload)
+    // ASDFFT_RAGGED_WIDE16 (measurement) asks for a form without the geometry by the longest class, which
+    // takes 79.9 us on the 4000-transform workload: =1 the EMAX-16 classes on wide workgroups (up to 1024
+    // threads per transform) in a launch of their own beside the single launch of the others (100.6 us),
+    // =0 one launch at the largest register budget (103.3 us)
     opt.wide16 = false;
     if (const char* w = getenv("ASDFFT_RAGGED_WIDE16")) {
         opt.wide16 = opt.one_launch && w[0] == '1';

@@ -11,8 +11,8 @@
 //
 // Each sample adds its frames in ascending order, as istft_ola_kernel does.
 //
-// The separate launches also write and read every frame (16 bytes a point): 122 us for 16
-// channels of 1000 frames of 1024 points at hop 256, 84 here.  VALU issue is 55% of that (65
+// The separate launches also write and read every frame (16 bytes a point): 118 us for 16
+// channels of 1000 frames of 1024 points at hop 256, 82.7 here.  VALU issue is 55% of that (65
 // instructions a point), the rest are the barriers of 16 wavefronts per CU: 16 frames of 1024
 // points with their tables fill the LDS.  16 frames are whole 128-byte lines of the spectrum;
 // groups of 8 with two workgroups per CU took 94 us.  With the later passes' twiddles in global

@@ -1664,7 +1664,7 @@ bool istft_two_launches_faster(const IstftFusedPlan& f, int64_t nfft, int64_t ch
 // group is 4 or 8 frames of it (26 x 440 x 939 hop 146: 83 us in groups of 4, 56 in groups of 16).
 // 128 VGPRs let 16 wavefronts share a CU, but three workgroups of five do not get onto its four
 // SIMDs together: planned as two, 9 x 700 x 1531 hop 175 86 -> 60 us, 12 x 720 x 363 hop 180 28 -> 22.
-// Separate launches -> one, us: 16 x 1024 x 1000 frames, hop 256 122 -> 82; 16 x 512 x 1000, hop 128
+// Separate launches -> one, us: 16 x 1024 x 1000 frames, hop 256 118 -> 83; 16 x 512 x 1000, hop 128
 // 67 -> 41; 12 x 720 x 500, hop 180 49 -> 32; 16 x 128 x 1000, hop 32 23 -> 12; 1 x 128 x 50 14.6 -> 11.
 bool build_istft_fused(const BuiltPlan& frames, int64_t nfft, int64_t channel, int64_t nframes, int64_t hop,
                        IstftFusedPlan* out)

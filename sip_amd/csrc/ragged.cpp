@@ -366,10 +366,11 @@ namespace {
 //     workgroups of 8 wavefronts per CU.  4000 transforms to 8192 50.1 -> 43.9 us, 2000 to 8192
 //     30.3 -> 25.8, 4000 to 4096 29.0 -> 27.2 against 32 points per thread, one workgroup per CU;
 //   * else every class on 1024 threads of up to 20 points, one workgroup of 16 wavefronts per CU
-//     (128 VGPRs): 4000 transforms to 16384 101.7 -> 84.2 us, 1000 33.4 -> 29.2, 300 26.4 -> 22.2
-//     against 48 points on 512 threads (79.9, 29.5, 19.4 with the exchange layout of RaggedRows;
-//     4000 to 8192 41.3, 2000 to 2048 on the EMAX-16 budget 13.2 -> 12.7).  The short classes in a
-//     launch of their own at half a CU take 90 us, after the long ones or beside them: the long tiles' last round is nearly empty;
+//     (128 VGPRs): 4000 transforms to 16384 105.2 -> 85.7 us, 1000 33.4 -> 29.1, 300 26.4 -> 22.2
+//     against 48 points on 512 threads.  The short classes in a launch of their own at half a CU take
+//     90 us, after the long ones or beside them: the long tiles' last round is nearly empty.  With the
+//     exchange layout of RaggedRows 79.9, 29.5 (level), 19.4; 4000 to 8192 41.3, 2000 to 2048 on the
+//     EMAX-16 budget 13.2 -> 12.7;
 //   * false where a class fits neither (13, 17, 19 in lengths near 16384): one launch at the largest
 //     register budget, as before.
 bool single_launch_geometry(const RaggedOptions& opt, std::vector<RaggedClassInfo>* classes)
